@@ -1,10 +1,11 @@
-// Residual encoders: one wavefront per token, lane L owns channels L and L+64.
+// Residual encoders: four lanes per token (eight for 4:16); inputs that are not
+// 16-byte aligned take one wavefront per token, lane L owning channels L and L+64.
 //
 // Every encoder computes r = f32(x) - f32(c[id]) and ranks channels by the
 // 15-bit magnitude of fp16(r) with ties going to the lower channel index
 // (reskv/csrc/compression.cu:80-118, 184-203, 287-313; reskv/compression.py:75-89).
-// The rank key is made unique by appending the inverted channel index, so
-// "top-k" is a single threshold on that composite key:
+// In the one-wavefront kernels the rank key is made unique by appending the
+// inverted channel index, so "top-k" is a single threshold on that composite key:
 //   ckey(d) = (|fp16(r_d)| bits) << 7 | (127 - d).
 // Top-k over all 128 channels uses a 22-step bitwise threshold search on
 // wave ballots; top-k inside a 16-channel tile counts larger keys from LDS.
@@ -243,37 +244,39 @@ __global__ void __launch_bounds__(256) encode_bitmap_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Unstructured top-nnz with MSB-first bitmaps, four lanes per token (lane
-// 4 t + q owns channels 32 q .. 32 q + 31 of token t; a wave encodes 16
-// tokens).  The nnz-th largest 15-bit magnitude M is found bit by bit on byte
-// planes: a lane's 32 magnitudes are split into a plane of high bytes (bits
-// 14..8) and one of low bytes, four values per dword, byte k of dword i
-// holding channel 32 q + 4 i + k.  A search step counts the bytes >= a
-// candidate c with two sums of absolute byte differences (v_sad_u8, against
-// c and c - 1), four values an instruction; the per-channel flags after each
-// phase use ((v | 0x80) - c) & 0x80, set exactly when v >= c (v, c <= 0x80,
-// no borrow crosses a byte).  Phases:
-//   A: the high seven bits H of M over the high bytes;
-//   B: bits 7..1 of M (L) over the low bytes >> 1 of the values whose high
-//      byte is H (the others read as 0 and never count: candidates are >= 1),
-//      on top of the count of values whose high byte exceeds H;
-//   C: bit 0 of M over the values whose high byte is H and low bits 7..1 are L.
-// Each step's count is summed over the token's four lanes (one quad) with two
-// DPP adds.  Channels above M are kept, and the lowest-indexed channels equal
-// to M fill the remainder (ties go to the lower channel, as with the
-// composite key).  The kept values are compacted into the wave's LDS rows and
-// written to the payload as 16-byte stores.
+// Selection on bit planes, four lanes per token (lane 4 t + q owns channels
+// 32 q .. 32 q + 31 of token t; a wave encodes 16 tokens).
+//
+// A lane's 32 fp16 residuals are transposed into bit planes: plane b holds bit
+// b of every magnitude, bit j of the plane being channel 32 q + j.  The k-th
+// largest magnitude is then found from the top plane down with one AND and one
+// popcount per plane for all 32 channels: `alive` are the channels that agree
+// with the threshold on the planes seen so far, and of these the ones with the
+// next bit set are either enough to hold the k-th largest (they stay alive) or
+// all above the threshold (they are kept, and the rest stays alive).  What is
+// alive after the last plane equals the threshold; ties go to the lower
+// channel.  The kept channels come out as a 32-bit mask, which is the metadata
+// word of the tile format and the reversed half word of the bitmaps.
+//
+// Bound: VALU issue.  The transpose takes 16 + 16 byte permutes and 96
+// shift / bit-select operations, the 15 planes about 12 instructions each,
+// against 224 byte-difference sums and about 260 instructions of sums, flags
+// and masks for the byte-plane search this replaced.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kByteTop = 0x80808080u;  // bit 7 of every byte
-constexpr uint32_t kByteOne = 0x01010101u;
-constexpr int kBitmapTokensPerWave = 16;
-constexpr int kBitmapDump = kBitmapTokensPerWave * kDim;  // per-wave LDS halves before the lanes' dump slots
+constexpr int kTokensPerWave = 16;
+constexpr int kTokensPerBlock = kWavesPerBlock * kTokensPerWave;
+constexpr int kRowPadHalves = 8;  // halves after each LDS payload row: 16-byte aligned rows that start on different banks
+constexpr int kRowHalves = kTokensPerWave * (kDim + kRowPadHalves);  // LDS halves of a wave's rows, before the dump slots
 
 // Sum over the four lanes of the lane's token (one DPP quad), in every one of them.
 __device__ __forceinline__ int quad_sum(int v) {
     v += (int)dpp_u<0xB1>((uint32_t)v);  // quad xor 1
     v += (int)dpp_u<0x4E>((uint32_t)v);  // quad xor 2
     return v;
+}
+__device__ __forceinline__ float quad_max(float v) {
+    v = fmaxf(v, dpp<0xB1>(v));
+    return fmaxf(v, dpp<0x4E>(v));
 }
 // Exclusive prefix sum over the quad, in lane (channel) order.
 __device__ __forceinline__ int quad_prefix(int v, int q) {
@@ -284,172 +287,365 @@ __device__ __forceinline__ int quad_prefix(int v, int q) {
     s += q >= 2 ? b : 0;
     return s - v;
 }
-// Bit-7 flags of the bytes of p (each ORed with 0x80 beforehand) that are >= the bytes of c4.
-__device__ __forceinline__ uint32_t ge_flags(uint32_t p, uint32_t c4) { return (p - c4) & kByteTop; }
-// Twice the number of the lane's 32 plane bytes (7-bit values, bit 7 clear)
-// that are >= the bytes of c4 (each 1..127), minus 32: for a byte a,
-// |a - c| - |a - (c - 1)| is -1 when a >= c and +1 otherwise, so two sums of
-// absolute byte differences (v_sad_u8, four bytes an instruction) give the
-// count without per-byte flags.
-__device__ __forceinline__ int twice_count_ge_minus(const uint32_t* p, uint32_t c4) {
-    uint32_t at = 0, below = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        at = __builtin_amdgcn_sad_u8(p[i], c4, at);
-        below = __builtin_amdgcn_sad_u8(p[i], c4 - kByteOne, below);
-    }
-    return (int)below - (int)at;  // = 2 * count - 32
-}
-// Largest 7-bit c (as four equal bytes) with base + (token count of plane bytes >= c) >= nnz,
-// over planes of 7-bit values.
-__device__ __forceinline__ uint32_t search7(const uint32_t* p, int base, int nnz) {
-    const int need = 2 * (nnz - base) - 4 * 32;  // 2 * count - 128 over the quad's 128 bytes
-    uint32_t c4 = 0;
-#pragma unroll
-    for (int bit = 6; bit >= 0; --bit) {
-        const uint32_t cand = c4 | (kByteOne << bit);
-        c4 = quad_sum(twice_count_ge_minus(p, cand)) >= need ? cand : c4;
-    }
-    return c4;
-}
-__global__ void __launch_bounds__(256) encode_bitmap4_kernel(EncSides S, int T, int nnz, int bh0) {
-    __shared__ __align__(16) uint16_t s_rows[kWavesPerBlock][kBitmapDump + kWave];
-    const int side = blockIdx.z;
-    const uint16_t* __restrict__ keys = S.x[side];
-    const uint16_t* __restrict__ cent = S.cent[side];
-    const int32_t* __restrict__ ids = S.ids[side];
-    uint16_t* __restrict__ payload = S.payload[side];
-    int64_t* __restrict__ meta = static_cast<int64_t*>(S.meta[side]);
-    const int C = S.C[side];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int q = lane & 3;
-    const int t_wave = blockIdx.x * (kWavesPerBlock * kBitmapTokensPerWave) + wave * kBitmapTokensPerWave;
-    if (t_wave >= T) return;  // whole waves
-    const int t = t_wave + (lane >> 2);
-    const bool valid = t < T;  // lanes past T compute on the last token and store nothing
-    const long bh = (long)bh0 + blockIdx.y;
-    const long row = bh * T + (valid ? t : T - 1);
+
+// The lane's 32 channels: tokens and centroid rows as loaded, residuals as fp16 pairs.
+struct Lane32 {
+    uint32_t x[16], c[16], h[16];  // channels 32 q + 2 i, + 1
+};
+__device__ __forceinline__ void load_lane32(const uint16_t* __restrict__ keys, const uint16_t* __restrict__ cent,
+                                            const int32_t* __restrict__ ids, long row, long bh, int C, int q,
+                                            Lane32& L) {
     int cid = ids[row];
     cid = cid < 0 ? 0 : (cid > C - 1 ? C - 1 : cid);  // compression.cu:83-84
     const uint4* xp = reinterpret_cast<const uint4*>(keys + row * kDim + q * 32);
     const uint4* cp = reinterpret_cast<const uint4*>(cent + (bh * C + cid) * kDim + q * 32);
-    uint32_t hp[16];  // fp16 residual pairs (channels 32 q + 2 i, + 1)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const uint4 xv = xp[j], cv = cp[j];
         const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w}, cw[4] = {cv.x, cv.y, cv.z, cv.w};
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            hp[4 * j + k] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, xw[k]) - __builtin_bit_cast(half2_t, cw[k]));
+        for (int k = 0; k < 4; ++k) {
+            L.x[4 * j + k] = xw[k];
+            L.c[4 * j + k] = cw[k];
+            L.h[4 * j + k] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, xw[k]) - __builtin_bit_cast(half2_t, cw[k]));
+        }
     }
-    // byte planes of the magnitudes (sign bits dropped): hr = bits 14..8, lb =
-    // bits 7..0; hb = hr with bit 7 of every byte set, for the flag tests
-    uint32_t hr[8], hb[8], lb[8];
+}
+
+__device__ __forceinline__ uint32_t bit_select(uint32_t m, uint32_t a, uint32_t b) { return (a & m) | (b & ~m); }
+
+// pl[b] = bit b of every channel's fp16 residual (bit j: channel j), b = 0..15.
+// Channels j and j + 16 share a dword, so the two 16 x 16 bit matrices in the
+// low and high halves are transposed together, in four exchange stages.
+__device__ __forceinline__ void bit_planes(const uint32_t* h, uint32_t* pl) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t m0 = hp[2 * i] & 0x7FFF7FFFu, m1 = hp[2 * i + 1] & 0x7FFF7FFFu;
-        hr[i] = __builtin_amdgcn_perm(m1, m0, 0x07050301u);
-        hb[i] = hr[i] | kByteTop;
-        lb[i] = __builtin_amdgcn_perm(m1, m0, 0x06040200u);
-    }
-    // A: high byte H of M
-    const uint32_t h4 = search7(hr, 0, nnz);
-    uint32_t gt_h[8], eq_h[8], l7r[8], l7[8];
-    int above = 0;
+    for (int j = 0; j < 16; ++j)
+        pl[j] = __builtin_amdgcn_perm(h[8 + (j >> 1)], h[j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        gt_h[i] = ge_flags(hb[i], h4 + kByteOne);  // H + 1 <= 0x80: no carry between bytes
-        eq_h[i] = ge_flags(hb[i], h4) & ~gt_h[i];
-        above += __builtin_popcount(gt_h[i]);
-        // bits 7..1 of the low byte where the high byte is H, else 0 (bytes of eq_h - (eq_h >> 7) are 0x7F or 0)
-        l7r[i] = (lb[i] >> 1) & (eq_h[i] - (eq_h[i] >> 7));
-        l7[i] = l7r[i] | kByteTop;
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t a = pl[j], b = pl[j + 8];
+        pl[j] = __builtin_amdgcn_perm(b, a, 0x06020400u);
+        pl[j + 8] = __builtin_amdgcn_perm(b, a, 0x07030501u);
     }
-    above = quad_sum(above);
-    // B: bits 7..1 of M
-    const uint32_t l4 = search7(l7r, above, nnz);
-    uint32_t gt_l[8], eq_l[8], one[8];
-    int above_l = 0, ones = 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        gt_l[i] = ge_flags(l7[i], l4 + kByteOne);            // high byte H, bits 7..1 above L
-        eq_l[i] = ge_flags(l7[i], l4) & ~gt_l[i] & eq_h[i];  // high byte H, bits 7..1 equal to L
-        one[i] = eq_l[i] & (lb[i] << 7);                      // ... with bit 0 set
-        above_l += __builtin_popcount(gt_l[i]);
-        ones += __builtin_popcount(one[i]);
-    }
-    above += quad_sum(above_l);
-    ones = quad_sum(ones);
-    // C: bit 0 of M
-    const bool m_odd = above + ones >= nnz;
-    const int need = nnz - (m_odd ? above : above + ones);  // ties to take, lowest channels first
-    uint32_t gt[8], eq[8];
-    int n_eq = 0;
+    for (int stage = 0; stage < 3; ++stage) {
+        const int s = 4 >> stage;
+        const uint32_t m = s == 4 ? 0x0F0F0F0Fu : (s == 2 ? 0x33333333u : 0x55555555u);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        gt[i] = gt_h[i] | gt_l[i] | (m_odd ? 0u : one[i]);
-        eq[i] = m_odd ? one[i] : eq_l[i] & ~one[i];
-        n_eq += __builtin_popcount(eq[i]);
+        for (int j = 0; j < 16; ++j) {
+            if (j & s) continue;
+            const uint32_t a = pl[j], b = pl[j + s];
+            pl[j] = bit_select(m, a, b << s);
+            pl[j + s] = bit_select(m, a >> s, b);
+        }
     }
-    int quota = need - quad_prefix(n_eq, q);
+}
+
+// Kept channels of the lane.  above: strictly larger than the threshold
+// magnitude; kept: those and the lowest-indexed ones equal to it.
+struct Kept {
+    uint32_t kept, above;
+};
+// Drops the highest-indexed of the equal channels until `quota` of them are left.
+__device__ __forceinline__ uint32_t lowest_bits(uint32_t eq, int quota) {
+    for (int n = __builtin_popcount(eq); n > quota; --n) eq &= ~(0x80000000u >> __builtin_clz(eq));
+    return eq;
+}
+// Top nnz of the token's 128 channels (1 <= nnz <= 128).
+__device__ __forceinline__ Kept select_token(const uint32_t* pl, int nnz, int q) {
+    uint32_t alive = 0xFFFFFFFFu, above = 0;
+    int need = nnz;
+#pragma unroll
+    for (int b = 14; b >= 0; --b) {
+        const uint32_t m = alive & pl[b];
+        const int n = quad_sum(__builtin_popcount(m));
+        const bool enough = n >= need;
+        above |= enough ? 0u : m;
+        alive = enough ? m : alive ^ m;
+        need = enough ? need : need - n;
+    }
+    int quota = need - quad_prefix(__builtin_popcount(alive), q);
     quota = quota < 0 ? 0 : quota;
-    while (n_eq > quota) {  // drop the highest-channel tie
-        int top = 0;
+    return Kept{above | lowest_bits(alive, quota), above};
+}
+// Top `per_tile` of each of the lane's two 16-channel tiles (the mask's halves).
+__device__ __forceinline__ uint32_t select_tiles(const uint32_t* pl, int per_tile) {
+    uint32_t alive = 0xFFFFFFFFu, above = 0;
+    int need0 = per_tile, need1 = per_tile;
 #pragma unroll
-        for (int i = 1; i < 8; ++i) top = eq[i] ? i : top;
-        uint32_t w = eq[0];
-#pragma unroll
-        for (int i = 1; i < 8; ++i) w = i == top ? eq[i] : w;
-        const uint32_t cleared = w & ~(0x80000000u >> __builtin_clz(w));
-#pragma unroll
-        for (int i = 0; i < 8; ++i) eq[i] = i == top ? cleared : eq[i];
-        --n_eq;
+    for (int b = 14; b >= 0; --b) {
+        const uint32_t m = alive & pl[b];
+        const int n0 = __builtin_popcount(m & 0xFFFFu), n1 = __builtin_popcount(m >> 16);
+        const bool e0 = n0 >= need0, e1 = n1 >= need1;
+        const uint32_t enough = (e0 ? 0xFFFFu : 0u) | (e1 ? 0xFFFF0000u : 0u);
+        above |= m & ~enough;
+        alive = bit_select(enough, m, alive ^ m);
+        need0 = e0 ? need0 : need0 - n0;
+        need1 = e1 ? need1 : need1 - n1;
     }
-    // kept channels as a 32-bit mask, bit i = channel 32 q + i: the flag bytes
-    // (0 or 1 after the shift) of two dwords weighted by 1..128 in one pair of
-    // byte dot products give 8 mask bits
-    uint32_t sel = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint32_t lo = (gt[2 * j] | eq[2 * j]) >> 7, hi = (gt[2 * j + 1] | eq[2 * j + 1]) >> 7;
-        const uint32_t m = __builtin_amdgcn_udot4(lo, 0x08040201u, __builtin_amdgcn_udot4(hi, 0x80402010u, 0u, false),
-                                                  false);
-        sel |= m << (8 * j);
+    return above | lowest_bits(alive & 0xFFFFu, need0) | lowest_bits(alive & 0xFFFF0000u, need1);
+}
+
+// Sparse FP16 formats.  TILE: top nnz / 8 of every 16-channel tile with
+// LSB-first tile masks; otherwise top nnz of the token with MSB-first bitmaps.
+// NNZ: the payload width when it is one of the common ones, else 0 (runtime).
+// The kept residuals go to the token's row in the wave's LDS in channel order
+// (the others to a dump slot of the lane, so the loop has no branch), and from
+// there to the payload as 16-byte stores.
+// 8 heads x 8192 tokens, K and V in one launch: 50% bitmap 18.7 -> 15.6 us, 75%
+// 17.9 -> 13.9 us (byte planes before), 50% tiles 41.2 -> 16.2 us (one wave per
+// token before).  64 heads x 16384 tokens: 231 -> 193, 210 -> 169 and 503 ->
+// 208 us, i.e. 4.4, 4.4 and 4.1 TB/s (a large copy reaches 4.9).
+template <bool TILE, int NNZ>
+__global__ void __launch_bounds__(256) encode_planes_kernel(EncSides S, int T, int nnz_arg, int bh0) {
+    __shared__ __align__(16) uint16_t s_rows[kWavesPerBlock][kRowHalves + kWave];
+    const int nnz = NNZ ? NNZ : nnz_arg;
+    const int side = blockIdx.z;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int q = lane & 3;
+    const int t_wave = blockIdx.x * kTokensPerBlock + wave * kTokensPerWave;
+    if (t_wave >= T) return;  // whole waves
+    const int t = t_wave + (lane >> 2);
+    const bool valid = t < T;  // lanes past T compute on the last token and store nothing
+    const long bh = (long)bh0 + blockIdx.y;
+    const long row = bh * T + (valid ? t : T - 1);
+    Lane32 L;
+    load_lane32(S.x[side], S.cent[side], S.ids[side], row, bh, S.C[side], q, L);
+    uint32_t pl[16];
+    bit_planes(L.h, pl);
+    const uint32_t sel = TILE ? select_tiles(pl, nnz >> 3) : select_token(pl, nnz, q).kept;
+    if constexpr (TILE) {
+        // word w = mask(tile 2w) | mask(tile 2w + 1) << 16
+        if (valid) static_cast<int32_t*>(S.meta[side])[row * 4 + q] = (int32_t)sel;
+    } else {
+        // channel d -> bit (63 - d % 64) of word d / 64 (compression.py:87-88):
+        // lane 2w holds the high half of word w, lane 2w + 1 the low half
+        const uint32_t rev = __builtin_bitreverse32(sel);
+        const uint32_t rev_next = dpp_u<0xB1>(rev);
+        if (valid && (q & 1) == 0)
+            static_cast<int64_t*>(S.meta[side])[row * 2 + (q >> 1)] = (int64_t)(((uint64_t)rev << 32) | rev_next);
     }
-    // the token keeps exactly nnz channels; the bound check keeps the LDS row
-    // writes inside the row regardless
     const int kept = __builtin_popcount(sel);
-    const int first = quad_prefix(kept, q);
-    if (first + kept > nnz) sel = 0;
-    // channel d -> bit (63 - d % 64) of word d / 64 (compression.py:87-88):
-    // lane 2w holds the high half of word w, lane 2w + 1 the low half
-    const uint32_t rev = __builtin_bitreverse32(sel);
-    const uint32_t rev_next = dpp_u<0xB1>(rev);
-    if (valid && (q & 1) == 0) meta[row * 2 + (q >> 1)] = (int64_t)(((uint64_t)rev << 32) | rev_next);
-    // payload: kept residuals in channel order into the token's LDS row (others
-    // to the lane's dump slot), then the wave's rows to HBM
+    const int first = TILE ? q * (nnz >> 2) : quad_prefix(kept, q);
+    const int pitch = nnz + kRowPadHalves;
     uint16_t* srow = s_rows[wave];
-    uint16_t* my_row = srow + (lane >> 2) * nnz;
-    uint16_t* dump = srow + kBitmapDump + lane;
-    int rank = first;
+    uint8_t* sbytes = reinterpret_cast<uint8_t*>(srow);
+    const uint32_t dump = 2 * (kRowHalves + lane);
+    int at = 2 * ((lane >> 2) * pitch + first + kept);  // byte offset past the lane's last kept value
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
-        const int bit = (int)((sel >> i) & 1u);
-        uint16_t* dst = bit ? my_row + rank : dump;
-        *dst = (uint16_t)(hp[i >> 1] >> (16 * (i & 1)));
-        rank += bit;
+    for (int i = 31; i >= 0; --i) {
+        const int m = __builtin_amdgcn_sbfe((int)sel, i, 1);  // -1 when channel i is kept
+        at += m * 2;
+        uint8_t* dst = sbytes + bit_select((uint32_t)m, (uint32_t)at, dump);
+        *reinterpret_cast<uint16_t*>(dst) = (uint16_t)(L.h[i >> 1] >> (16 * (i & 1)));
     }
     wave_sync();
-    const int ntok = T - t_wave < kBitmapTokensPerWave ? T - t_wave : kBitmapTokensPerWave;
-    uint16_t* grow = payload + (bh * T + t_wave) * (long)nnz;  // the wave's rows are contiguous
-    const int halves = ntok * nnz;
+    const int ntok = T - t_wave < kTokensPerWave ? T - t_wave : kTokensPerWave;
+    uint16_t* grow = S.payload[side] + (bh * T + t_wave) * (long)nnz;  // the wave's rows are contiguous
     if ((nnz & 7) == 0) {
-        const uint4* src = reinterpret_cast<const uint4*>(srow);
+        const int per = nnz >> 3;
         uint4* dst = reinterpret_cast<uint4*>(grow);
-        for (int c = lane; c < halves / 8; c += kWave) dst[c] = src[c];
+        for (int c = lane; c < ntok * per; c += kWave) {
+            const int r = c / per;
+            dst[c] = *reinterpret_cast<const uint4*>(srow + r * pitch + 8 * (c - r * per));
+        }
     } else {
-        for (int c = lane; c < halves; c += kWave) grow[c] = srow[c];
+        for (int c = lane; c < ntok * nnz; c += kWave) {
+            const int r = c / nnz;
+            grow[c] = srow[r * pitch + c - r * nnz];
+        }
     }
+}
+
+// ---------------------------------------------------------------------------
+// Unstructured top-nnz with INT4 / INT2 codes (compression.cu:245-383), on the
+// same planes.  With s the fp16-rounded scale, a code is
+// clamp(rint(fl32(r / s)), -QMAX, QMAX).  It is formed without a division per
+// channel, exactly:
+//   INT2: rint(fl32(r / s)) is 0 exactly when |r| <= s / 2.  (s / 2 and the
+//   other rounding boundaries b s, b = k + 1/2 <= 7.5, have at most 15
+//   significant bits, so they are exact in fp32; if r is not b s, r / s differs
+//   from b by at least ulp(b) / m with m the significand of s, 1 <= m < 2, so
+//   that fl32(r / s) is not b either.)
+//   INT4: t = r * rcp(s) plus one Newton correction is within 2^-20 ulp of r / s
+//   before its last rounding, while the quotients nearest a boundary are at
+//   least 0.0002 ulp away from rounding to it: rint gives the same integer.
+//   Adding 1.5 * 2^23 rounds to the nearest even integer in the low bits, and
+//   eight codes biased by 8 are gathered by shift-adds.
+// Waves in which a residual is infinite or NaN, a scale is zero or infinite,
+// or every kept magnitude ties (the largest |r| in fp32 may then be among the
+// dropped channels) take the plain form: the masked maximum, and a division
+// per channel.
+// K and V of 64 heads x 16384 tokens at 50%: INT4 681 -> 172 us (4.0 TB/s), INT2
+// 728 -> 148 us (4.2 TB/s), against the one-wave-per-token kernels, which take
+// four lanes' ballots for each of 22 search steps and divide for every channel.
+// ---------------------------------------------------------------------------
+template <int BITS>
+__global__ void __launch_bounds__(256) encode_quant_kernel(const uint16_t* __restrict__ keys,
+                                                           const uint16_t* __restrict__ cent,
+                                                           const int32_t* __restrict__ ids,
+                                                           uint32_t* __restrict__ qtiles,
+                                                           uint16_t* __restrict__ qscale, int T, int C, int nnz,
+                                                           int bh0) {
+#pragma clang fp contract(off)
+    constexpr int kQmax = (1 << (BITS - 1)) - 1;
+    constexpr int kPerWord = 32 / BITS;
+    constexpr int kLaneWords = BITS;  // 32 channels of BITS bits
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int q = lane & 3;
+    const int t_wave = blockIdx.x * kTokensPerBlock + wave * kTokensPerWave;
+    if (t_wave >= T) return;  // whole waves
+    const int t = t_wave + (lane >> 2);
+    const bool valid = t < T;  // lanes past T compute on the last token and store nothing
+    const long bh = (long)bh0 + blockIdx.y;
+    const long row = bh * T + (valid ? t : T - 1);
+    Lane32 L;
+    load_lane32(keys, cent, ids, row, bh, C, q, L);
+    uint32_t pl[16];
+    bit_planes(L.h, pl);
+    const Kept K = select_token(pl, nnz, q);
+    const uint32_t sel = K.kept;
+    float r[32];
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        const uint32_t sh = 16u * (i & 1);
+        r[i] = h2f((uint16_t)(L.x[i >> 1] >> sh)) - h2f((uint16_t)(L.c[i >> 1] >> sh));
+        amax = fmaxf(amax, fabsf(r[i]));
+    }
+    amax = quad_max(amax);
+    // fp16(amax / QMAX) with an IEEE fp32 division, fp16(1) for an all-zero residual
+    uint16_t hs = amax > 0.0f ? f2h(amax / (float)kQmax) : f2h(1.0f);
+    const uint32_t nonfinite = pl[14] & pl[13] & pl[12] & pl[11] & pl[10];
+    const int above = quad_sum(__builtin_popcount(K.above));
+    const bool plain = nonfinite != 0 || above == 0 || (hs & 0x7FFFu) == 0 || hs >= 0x7C00u;
+    uint32_t w[kLaneWords];
+    if (ballot(plain) == 0) {
+        const float sf = h2f(hs);
+        if constexpr (BITS == 2) {
+            const float half_step = 0.5f * sf;
+            uint32_t nz = 0, neg = 0;  // bit i: channel i has a nonzero code / is negative
+#pragma unroll
+            for (int i = 31; i >= 0; --i) {
+                nz = __builtin_amdgcn_alignbit(nz, (uint32_t)f2i(half_step - fabsf(r[i])), 31);
+                neg = __builtin_amdgcn_alignbit(neg, (uint32_t)f2i(r[i]), 31);
+            }
+            nz &= sel;
+            neg &= nz;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                uint32_t a = (nz >> (16 * k)) & 0xFFFFu, n = (neg >> (16 * k)) & 0xFFFFu;
+#pragma unroll
+                for (int stage = 0; stage < 4; ++stage) {  // bit i to bit 2 i
+                    const int s = 8 >> stage;
+                    const uint32_t m = s == 8 ? 0x00FF00FFu : (s == 4 ? 0x0F0F0F0Fu : (s == 2 ? 0x33333333u : 0x55555555u));
+                    a = (a | (a << s)) & m;
+                    n = (n | (n << s)) & m;
+                }
+                w[k] = a | (n << 1);  // 01: +1, 11: -1
+            }
+        } else {
+            const float inv = __builtin_amdgcn_rcpf(sf);
+            constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23, bits 0x4B400000
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                uint32_t acc = 0;
+#pragma unroll
+                for (int j = 7; j >= 0; --j) {
+                    const float v = r[8 * k + j];
+                    float d = v * inv;
+                    d = __builtin_fmaf(__builtin_fmaf(-d, sf, v), inv, d);
+                    d = __builtin_amdgcn_fmed3f(d, -7.0f, 7.0f);
+                    acc = (acc << 4) + (uint32_t)f2i(d + kMagic);
+                }
+                acc = (acc - 0x4B400000u * 0x11111111u + 0x88888888u) ^ 0x88888888u;
+                // the kept channels' nibbles
+                uint32_t m = (sel >> (8 * k)) & 0xFFu;
+                m = (m | (m << 12)) & 0x000F000Fu;
+                m = (m | (m << 6)) & 0x03030303u;
+                m = (m | (m << 3)) & 0x11111111u;
+                w[k] = acc & ((m << 4) - m);
+            }
+        }
+    } else {
+        amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) amax = fmaxf(amax, (sel >> i) & 1u ? fabsf(r[i]) : 0.0f);
+        amax = quad_max(amax);
+        hs = amax > 0.0f ? f2h(amax / (float)kQmax) : f2h(1.0f);
+        const float sf = h2f(hs);
+#pragma unroll
+        for (int k = 0; k < kLaneWords; ++k) {
+            uint32_t acc = 0;
+#pragma unroll
+            for (int j = 0; j < kPerWord; ++j) {
+                int code = (int)rintf(r[kPerWord * k + j] / sf);
+                code = code < -kQmax ? -kQmax : (code > kQmax ? kQmax : code);
+                if ((sel >> (kPerWord * k + j)) & 1u) acc |= (uint32_t)(code & ((1 << BITS) - 1)) << (BITS * j);
+            }
+            w[k] = acc;
+        }
+    }
+    if (!valid) return;
+    uint32_t* dst = qtiles + row * (4 * kLaneWords) + kLaneWords * q;
+    if constexpr (BITS == 4) *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
+    else *reinterpret_cast<uint2*>(dst) = make_uint2(w[0], w[1]);
+    if (q == 0) qscale[row] = hs;
+}
+
+// ---------------------------------------------------------------------------
+// Structured INT4 (compression.cu:153-239): 1 of every 4 channels, four lanes
+// per token as above (lane q: subgroups 8 q .. 8 q + 7, i.e. payload word q and
+// half a metadata word), so every load and store is a contiguous run.  K and V
+// of 64 heads x 16384 tokens: 541 -> 128 us, 4.8 TB/s, the rate of a large copy.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) encode_sint4_kernel(const uint16_t* __restrict__ keys,
+                                                           const uint16_t* __restrict__ cent,
+                                                           const int32_t* __restrict__ ids,
+                                                           int32_t* __restrict__ qpacked, int32_t* __restrict__ qmeta,
+                                                           uint16_t* __restrict__ qscale, int T, int C, int bh0) {
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int q = lane & 3;
+    const int t_wave = blockIdx.x * kTokensPerBlock + wave * kTokensPerWave;
+    if (t_wave >= T) return;  // whole waves
+    const int t = t_wave + (lane >> 2);
+    const bool valid = t < T;  // lanes past T compute on the last token and store nothing
+    const long bh = (long)bh0 + blockIdx.y;
+    const long row = bh * T + (valid ? t : T - 1);
+    Lane32 L;
+    load_lane32(keys, cent, ids, row, bh, C, q, L);
+    float v[8];
+    uint32_t pos_bits = 0;
+    float amax = 0.0f;
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+        // largest |fp16(r)| of the four, the lower channel on ties: magnitude
+        // above the inverted position
+        const uint32_t a = L.h[2 * g], b = L.h[2 * g + 1];
+        const uint32_t k0 = ((a & 0x7FFFu) << 2) | 3u, k1 = ((a >> 14) & 0x1FFFCu) | 2u;
+        const uint32_t k2 = ((b & 0x7FFFu) << 2) | 1u, k3 = (b >> 14) & 0x1FFFCu;
+        const uint32_t pos = 3u - (max(max(k0, k1), max(k2, k3)) & 3u);
+        const uint32_t xw = pos & 2u ? L.x[2 * g + 1] : L.x[2 * g], cw = pos & 2u ? L.c[2 * g + 1] : L.c[2 * g];
+        const uint32_t sh = (pos & 1u) * 16u;
+        v[g] = h2f((uint16_t)(xw >> sh)) - h2f((uint16_t)(cw >> sh));
+        amax = fmaxf(amax, fabsf(v[g]));
+        pos_bits |= pos << (2 * g);
+    }
+    amax = quad_max(amax);
+    const float s = amax > 0.0f ? amax * (1.0f / 7.0f) : 1.0f;  // compression.cu:224
+    uint32_t word = 0;
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+        int code = (int)rintf(v[g] / s);
+        code = code < -7 ? -7 : (code > 7 ? 7 : code);
+        word |= (uint32_t)(code & 0xF) << (4 * g);
+    }
+    const uint32_t pos_next = dpp_u<0xB1>(pos_bits);  // quad xor 1: the other half of the metadata word
+    if (!valid) return;
+    qpacked[row * 4 + q] = (int32_t)word;
+    if ((q & 1) == 0) qmeta[row * 2 + (q >> 1)] = (int32_t)(pos_bits | (pos_next << 16));
+    if (q == 0) qscale[row] = f2h(s);
 }
 
 template <int BITS>
@@ -577,21 +773,31 @@ int launch_tile4(const EncSides& S, int sides, int B, int H, int T, int struct_i
     return reskv_host::check_launch("encode_tile4_kernel");
 }
 
-// bitmap fast path: 16-byte aligned tokens, centroids and payload.
-bool bitmap4_ok(const EncSides& S, int sides) {
+// four-lanes-per-token encoders: 16-byte aligned tokens, centroids and payload.
+bool planes_ok(const EncSides& S, int sides) {
     bool ok = true;
     for (int i = 0; i < sides; ++i) ok = ok && aligned16(S.x[i]) && aligned16(S.cent[i]) && aligned16(S.payload[i]);
     return ok;
 }
-int launch_bitmap4(const EncSides& S, int sides, int B, int H, int T, int nnz, hipStream_t st) {
-    const int BH = B * H;
-    const int per_block = kWavesPerBlock * kBitmapTokensPerWave;
-    for (int bh0 = 0; bh0 < BH; bh0 += 65535) {  // grid y covers at most 65535 (batch, head) rows
-        const dim3 grid((T + per_block - 1) / per_block, BH - bh0 < 65535 ? BH - bh0 : 65535, sides);
-        hipLaunchKernelGGL(encode_bitmap4_kernel, grid, dim3(256), 0, st, S, T, nnz, bh0);
-        if (reskv_host::check_launch("encode_bitmap4_kernel")) return 1;
+// Calls launch(grid, first (batch, head) row) over all rows: grid y covers at most 65535 of them.
+template <typename Launch>
+int over_rows(int BH, int T, int sides, const char* what, Launch launch) {
+    for (int bh0 = 0; bh0 < BH; bh0 += 65535) {
+        launch(dim3((T + kTokensPerBlock - 1) / kTokensPerBlock, BH - bh0 < 65535 ? BH - bh0 : 65535, sides), bh0);
+        if (reskv_host::check_launch(what)) return 1;
     }
     return 0;
+}
+template <bool TILE>
+int launch_planes(const EncSides& S, int sides, int B, int H, int T, int nnz, hipStream_t st) {
+    return over_rows(B * H, T, sides, "encode_planes_kernel", [&](dim3 grid, int bh0) {
+        if (nnz == 64)
+            hipLaunchKernelGGL((encode_planes_kernel<TILE, 64>), grid, dim3(256), 0, st, S, T, nnz, bh0);
+        else if (nnz == 32)
+            hipLaunchKernelGGL((encode_planes_kernel<TILE, 32>), grid, dim3(256), 0, st, S, T, nnz, bh0);
+        else
+            hipLaunchKernelGGL((encode_planes_kernel<TILE, 0>), grid, dim3(256), 0, st, S, T, nnz, bh0);
+    });
 }
 
 }  // namespace
@@ -608,6 +814,7 @@ extern "C" int reskv_compress_fp16(const void* keys, const void* centroids, cons
     const EncSides S{{(const uint16_t*)keys, nullptr}, {(const uint16_t*)centroids, nullptr}, {ids, nullptr},
                      {(uint16_t*)payload, nullptr}, {meta, nullptr}, {C, 0}};
     if (tile4_ok(S, 1, nnz)) return launch_tile4(S, 1, B, H, T, struct_index, (hipStream_t)stream);
+    if (planes_ok(S, 1)) return launch_planes<true>(S, 1, B, H, T, nnz, (hipStream_t)stream);
     hipLaunchKernelGGL(encode_qtile_kernel, dim3(grid_for(rows)), dim3(256), 0, (hipStream_t)stream,
                        (const uint16_t*)keys, (const uint16_t*)centroids, ids, (uint16_t*)payload, meta,
                        rows, T, C, nnz, struct_index);
@@ -623,7 +830,7 @@ extern "C" int reskv_compress_bitmap(const void* keys, const void* centroids, co
     const long rows = (long)B * H * T;
     const EncSides S{{(const uint16_t*)keys, nullptr}, {(const uint16_t*)centroids, nullptr}, {ids, nullptr},
                      {(uint16_t*)payload, nullptr}, {meta, nullptr}, {C, 0}};
-    if (bitmap4_ok(S, 1)) return launch_bitmap4(S, 1, B, H, T, nnz, (hipStream_t)stream);
+    if (planes_ok(S, 1)) return launch_planes<false>(S, 1, B, H, T, nnz, (hipStream_t)stream);
     hipLaunchKernelGGL(encode_bitmap_kernel, dim3(grid_for(rows)), dim3(256), 0, (hipStream_t)stream,
                        (const uint16_t*)keys, (const uint16_t*)centroids, ids, (uint16_t*)payload, meta,
                        rows, T, C, nnz);
@@ -638,6 +845,13 @@ extern "C" int reskv_compress_quantized(const void* keys, const void* centroids,
     RESKV_REQUIRE(nnz == 32 || nnz == 64, "quantised encoder requires nnz in {32, 64}");
     RESKV_REQUIRE(bits == 2 || bits == 4, "quantised encoder requires bits in {2, 4}");
     const long rows = (long)B * H * T;
+    // rows read and written with 16-byte (INT2: 8-byte) accesses where they are aligned to them
+    if (aligned16(keys) && aligned16(centroids) && aligned16(qtiles))
+        return over_rows(B * H, T, 1, "encode_quant_kernel", [&](dim3 grid, int bh0) {
+            auto kernel = bits == 4 ? encode_quant_kernel<4> : encode_quant_kernel<2>;
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)keys,
+                               (const uint16_t*)centroids, ids, (uint32_t*)qtiles, (uint16_t*)qscale, T, C, nnz, bh0);
+        });
     if (bits == 4)
         hipLaunchKernelGGL(encode_multibit_kernel<4>, dim3(grid_for(rows)), dim3(256), 0, (hipStream_t)stream,
                            (const uint16_t*)keys, (const uint16_t*)centroids, ids, qtiles,
@@ -655,6 +869,11 @@ extern "C" int reskv_compress_structured_int4(const void* keys, const void* cent
     if (check_common(keys, centroids, ids, B, H, T, C)) return 1;
     RESKV_REQUIRE(qpacked && qmeta && qscale, "null output pointer");
     const long rows = (long)B * H * T;
+    if (aligned16(keys) && aligned16(centroids))
+        return over_rows(B * H, T, 1, "encode_sint4_kernel", [&](dim3 grid, int bh0) {
+            hipLaunchKernelGGL(encode_sint4_kernel, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)keys,
+                               (const uint16_t*)centroids, ids, qpacked, qmeta, (uint16_t*)qscale, T, C, bh0);
+        });
     hipLaunchKernelGGL(encode_struct_int4_kernel, dim3(grid_for(rows)), dim3(256), 0, (hipStream_t)stream,
                        (const uint16_t*)keys, (const uint16_t*)centroids, ids, qpacked, qmeta,
                        (uint16_t*)qscale, rows, T, C);
@@ -675,6 +894,8 @@ extern "C" int reskv_compress_fp16_kv(const void* k, const void* v, const void* 
                      {k_ids, v_ids}, {(uint16_t*)k_payload, (uint16_t*)v_payload}, {k_meta, v_meta}, {Ck, Cv}};
     if (tile4_ok(S, 2, nnz) && (!struct_index || nnz == 32))
         return launch_tile4(S, 2, B, H, T, struct_index, (hipStream_t)stream);
+    if (planes_ok(S, 2) && !struct_index && nnz > 0 && nnz < kDim && nnz % 8 == 0)
+        return launch_planes<true>(S, 2, B, H, T, nnz, (hipStream_t)stream);
     if (reskv_compress_fp16(k, k_centroids, k_ids, k_payload, k_meta, B, H, T, Ck, nnz, struct_index, stream))
         return 1;
     return reskv_compress_fp16(v, v_centroids, v_ids, v_payload, v_meta, B, H, T, Cv, nnz, struct_index, stream);
@@ -690,7 +911,7 @@ extern "C" int reskv_compress_bitmap_kv(const void* k, const void* v, const void
     RESKV_REQUIRE(nnz > 0 && nnz <= kDim, "nnz must be in [1, 128]");
     const EncSides S{{(const uint16_t*)k, (const uint16_t*)v}, {(const uint16_t*)k_centroids, (const uint16_t*)v_centroids},
                      {k_ids, v_ids}, {(uint16_t*)k_payload, (uint16_t*)v_payload}, {k_meta, v_meta}, {Ck, Cv}};
-    if (bitmap4_ok(S, 2)) return launch_bitmap4(S, 2, B, H, T, nnz, (hipStream_t)stream);
+    if (planes_ok(S, 2)) return launch_planes<false>(S, 2, B, H, T, nnz, (hipStream_t)stream);
     if (reskv_compress_bitmap(k, k_centroids, k_ids, k_payload, k_meta, B, H, T, Ck, nnz, stream)) return 1;
     return reskv_compress_bitmap(v, v_centroids, v_ids, v_payload, v_meta, B, H, T, Cv, nnz, stream);
 }
