@@ -11,7 +11,9 @@
 // iteration): each fp32 centre is split into fp16 hi + lo rows, stored with
 // |c|^2, padded to a multiple of 16 rows (padding rows are zero with an
 // infinite norm).  They are written once per iteration, so the assignment
-// workgroups load ready matrix-core operands instead of rebuilding them.
+// workgroups load ready matrix-core operands instead of rebuilding them.  The
+// fp16 norms of the V tokens, which the V rule needs in every iteration, are
+// written by the first one.
 //
 // Assignment (kmeans_assign_kernel): the distance GEMM S^T = C X^T runs on the
 // matrix cores (v_mfma_f32_16x16x32f16).  Tokens are fp16 already and
@@ -26,18 +28,16 @@
 //     fp16(|x|^2_h + |c|^2_h - 2 <x, c>), clamped at zero, square-rooted to
 //     fp16; |.|^2_h is the fp16 sum of fp16-rounded squares;
 //   V, decode groups (compression.py:61-64):
-//     fp16(|x|^2_h + |c|^2_h) - 2 <x, c> in fp32.  Member sums are a second matrix-core
-// product, onehot(ids)^T X, whose X operand comes from the wave's 16-token tile
-// through LDS transpose reads; the member counts are the same product against
-// an all-ones operand.  One-hot entries and tokens are exact in fp16 and the
-// products accumulate in fp32.  The waves of a chunk write their sums to
-// separate LDS regions that are added in a fixed order, so sums, counts and
-// centres are deterministic.
-// Update (kmeans_update_kernel): one workgroup per (cluster, problem) reduces
-// the chunk partials in a fixed order, writes the new centre and its tables.
+//     fp16(|x|^2_h + |c|^2_h) - 2 <x, c> in fp32.
+// Member sums are a second matrix-core product, onehot(ids)^T X, whose X operand
+// comes from the staged token rows through LDS transpose reads.  One-hot entries
+// and tokens are exact in fp16 and the products accumulate in fp32, in an order
+// that does not depend on the launch; counts are integer LDS adds.  Sums, counts
+// and centres are deterministic, and equal for paired and separate runs.
+// Update (kmeans_update_kernel): one workgroup per (cluster, problem) adds the
+// partials in a fixed order, writes the new centre and its tables.
 #include "common.h"
 #include "../../include/reskv_hip.h"
-
 using namespace reskv;
 
 namespace {
@@ -48,23 +48,11 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_t lds_short4_t;
 
-constexpr int kWaves = 8;
-constexpr int kRegions = 4;  // LDS sum regions: waves w and w + 4 share region w
-constexpr int kThreads = kWaves * kWave;
 constexpr int kSub = 16;           // tokens per MFMA sub-tile
-constexpr int kChunk = 256;        // tokens per assignment workgroup (two sub-tiles per wave)
+constexpr int kChunk = 256;        // tokens per chunk of the member sums
 constexpr int kCUs = 256;          // compute units of an MI355X
 constexpr int kXPitch = kDim + 8;  // halves per staged token row (16-byte aligned rows)
-constexpr int kRPitch = kDim + 4;  // floats per cluster row of a wave's sum region; column kDim is the count
-
-template <int NB>
-constexpr int region_floats() { return NB * 16 * kRPitch; }
-template <int NB>
-constexpr int smem_bytes() {
-    const int loop = kWaves * kSub * kXPitch * 2 + (NB > 2 ? 2 * NB * 16 * kDim * 2 : 0);
-    const int reduce = kRegions * region_floats<NB>() * 4;
-    return loop > reduce ? loop : reduce;
-}
+constexpr int kParts = 4;          // interleaved parts of a problem's chunk sums (chunk k belongs to part k % 4)
 
 __device__ __forceinline__ half8_t as_h8(uint4 v) { return __builtin_bit_cast(half8_t, v); }
 
@@ -157,6 +145,15 @@ __global__ void __launch_bounds__(kDim) kmeans_prep_rows_kernel(Problems P, Init
     store_tables(v, true, pad, bh >= P.vfrom, c, thi + head, tlo + head, tnorm + bh * Cp + c, s_w);
 }
 
+// Four fp16 values, 2.0 where a byte of id4 equals the byte repeated in `mine`
+// and 0 elsewhere.  All bytes are below 64: 0x40 - byte keeps bit 6 exactly for a
+// zero difference and never borrows from the next byte, and 0x4000 is fp16 2.0.
+__device__ __forceinline__ half4_t one_hot4(uint32_t id4, uint32_t mine) {
+    const uint32_t e = (0x40404040u - (id4 ^ mine)) & 0x40404040u;
+    return __builtin_bit_cast(half4_t, make_uint2(__builtin_amdgcn_perm(0u, e, 0x010C000Cu),
+                                                  __builtin_amdgcn_perm(0u, e, 0x030C020Cu)));
+}
+
 // |c|^2 of centre r of a lane's four
 __device__ __forceinline__ float cnorm(float4 n, int r) { return r == 0 ? n.x : r == 1 ? n.y : r == 2 ? n.z : n.w; }
 
@@ -232,126 +229,186 @@ __device__ __forceinline__ float root_bound_sq(float d) {
     return m * m;
 }
 
-// One workgroup: tokens [chunk * kChunk, +kChunk) of problem bh; wave w takes
-// sub-tiles w and w + 8 of the chunk, loaded together at the start.
+// Work split of the assignment over a workgroup's waves.  A chunk's 16 sub-tiles
+// are summed as r_j = S_{j+4} + S_j, j = 0..3, S_w being sub-tile w, then w + 8; the
+// four sub-tiles of an r_j are staged and summed together.  A group of waves works
+// on JU of them at a time, one sub-tile per wave; for the member sums its waves
+// split the channels in four and, for more than 32 centres, the centre blocks in
+// two.  G = 4 groups share a chunk, or one group (G = 1) takes all four r_j in turn.
+template <int NB, int G>
+struct Split {
+    static constexpr int JU = NB <= 2 ? 1 : 2;
+    static constexpr int GW = 4 * JU;                 // waves per group
+    static constexpr int MB = (NB + JU - 1) / JU;     // centre blocks per wave in the member sums
+    static constexpr int NH = 2;                      // 16-channel blocks per wave
+    static constexpr int US = 4 * JU;                 // sub-tiles per unit
+    static constexpr int waves = GW * G, threads = kWave * waves;
+    static constexpr int turns = 4 / (JU * G);        // units of a chunk that a group takes
+    static_assert(JU * G * turns == 4 && (G == 1 || JU == 1), "the four r_j of a chunk");
+};
+// Sub-tile e of r_j (order of summation).
+__device__ __forceinline__ int sub_of(int j, int e) { return j + (e < 2 ? 4 : 0) + (e & 1 ? 8 : 0); }
+
+// One workgroup: chunks slot, slot + slots, ... of problem bh (256 tokens each).
+//
+// Per unit: the wave's sub-tile of token rows goes from its registers to LDS and,
+// with the centre operands in LDS, through the distance products; the registers
+// then take the next sub-tile's rows, requested before the ids are found, so that
+// the loads have the rest of the unit to arrive.  After a barrier the group forms its member
+// sums over the unit, each wave for its own channels and centres, so that a sum
+// never leaves its lane: no reduction over waves.  The one-hot operand is made from
+// four id bytes at a time (2.0 = 0x4000 where a byte equals the lane's cluster; the
+// doubled sums are exact and halved at the end).
+// Sums are formed in one fixed order whatever slots and G are: r_j as above,
+// ((r_0 + r_1) + r_2) + r_3 per chunk, and the chunks of one part (k % 4) in
+// increasing order.  A workgroup therefore takes one chunk or a whole part (slots = 4).
+//
 // thi/tlo fp16 [BH, 16 NB, 128] and tnorm fp32 [BH, 16 NB] are the centre
-// tables; psum fp32 [BH, chunks, C, 128] and pcnt int [BH, chunks, C] (skipped
-// when psum is null).  LO: some problem has fp32 centres (lo tables of the
-// others are zero).  REGB: centre operands held in registers (one workgroup per
-// CU); otherwise read from LDS, which frees the registers for two workgroups
-// per CU (four waves per SIMD: at most 128 VGPRs, requested from the compiler
-// with waves_per_eu) when the grid has more workgroups than CUs.  At three
-// waves per SIMD only one 8-wave workgroup fits and K+V together at 512
-// workgroups took 290 us instead of 245 us.
-template <int NB, bool LO, bool REGB>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(REGB ? 1 : 4)))
+// tables; psum fp32 [BH, slots, C, 128] and pcnt int [BH, slots, C] (skipped
+// when psum is null).  xnorm (null: formed in place) holds the V tokens' fp16
+// norms [V problems, T]: written when xnorm_new, read otherwise.  LO: some
+// problem has fp32 centres (V problems skip the lo product).
+//
+// Bound: reading the rows and the VALU work (argmin, one-hot operands) take about
+// 0.1 ms each per iteration of 256 problems x 8128 tokens and overlap through four
+// independent four-wave workgroups per CU (128 VGPRs, 34 KB of LDS).  The whole
+// K-means of that size, 10 iterations: 2330 -> 1556 us; 16 problems x 8192: 214 ->
+// 184 us; 48 problems x 1999, C = 48, 15 iterations: 444 -> 329 us.  The kernel
+// before had eight waves reduce 16 KB sums each through LDS for every chunk, wrote
+// a 16 KB partial per 64 KB of tokens, and (C > 32) fitted one workgroup per CU.
+template <int NB, bool LO, int G>
+__global__ void __launch_bounds__((Split<NB, G>::threads)) __attribute__((amdgpu_waves_per_eu(4)))
 kmeans_assign_kernel(
     Problems P, const uint16_t* __restrict__ thi, const uint16_t* __restrict__ tlo, const float* __restrict__ tnorm,
-    float* __restrict__ psum, int* __restrict__ pcnt, int T, int C, int chunks) {
-    constexpr int CP = NB * 16;
-    constexpr int SPW = kChunk / (kWaves * kSub);  // sub-tiles per wave
-    constexpr bool kRegB = REGB && NB <= 2;
-    __shared__ __align__(16) unsigned char smem[smem_bytes<NB>()];
-    const int chunk = blockIdx.x;
+    float* __restrict__ psum, int* __restrict__ pcnt, float* __restrict__ xnorm, int xnorm_new, int T, int C,
+    int chunks) {
+    using W = Split<NB, G>;
+    constexpr int CP = NB * 16, MB = W::MB, NH = W::NH, JU = W::JU, US = W::US;
+    constexpr int kTab = CP * kDim / 8;                 // 16-byte slots of a centre table
+    constexpr int kRows = US * kSub * kXPitch;          // halves of a group's staged rows
+    constexpr int kSumFloats = CP * kDim;
+    constexpr int kSumBytes = G > 1 ? 3 * kSumFloats * 4 : 0;  // r_j handed to group 0 (reuses the rows)
+    constexpr int kRowBytes = G * kRows * 2 > kSumBytes ? G * kRows * 2 : kSumBytes;
+    __shared__ __align__(16) uint8_t s_rows[kRowBytes];
+    __shared__ __align__(16) uint4 s_hi[kTab];
+    __shared__ __align__(16) uint4 s_lo[LO ? kTab : 1];
+    __shared__ __align__(16) uint8_t s_id[G * US * kSub];
+    __shared__ int s_cnt[CP];
+    const int slot = blockIdx.x, slots = gridDim.x;
     const long bh = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int col = lane & 15, grp = lane >> 4;  // MFMA lane coordinates
-    uint16_t* xs = reinterpret_cast<uint16_t*>(smem) + wave * kSub * kXPitch;
+    const int g = wave / W::GW, gw = wave % W::GW;  // group, wave of the group
+    const int col = lane & 15, grp = lane >> 4;     // MFMA lane coordinates
     const int side = side_of(P, bh);
     const long pb = bh - (side ? P.split : 0);
     const uint16_t* __restrict__ x = P.x[side] + pb * T * kDim;
     int32_t* __restrict__ ids = P.ids[side] + pb * T;
     const bool vrule = bh >= P.vfrom;  // workgroup-uniform
     const bool vgroup = P.vgroup != 0;
+    float* __restrict__ xn_row = vrule && xnorm != nullptr ? xnorm + (bh - P.vfrom) * T : nullptr;
+    uint16_t* s_x = reinterpret_cast<uint16_t*>(s_rows) + g * kRows;
+    uint8_t* g_id = s_id + g * US * kSub;
 
     // token operand: lane (col, grp) holds token t0 + col, channels 32 q + 8 grp +
-    // [0, 8) for piece q, so the four lanes of a token read 64 contiguous bytes;
-    // rows past T repeat token t0 (their one-hot entries are 0)
-    uint4 xr[SPW][4];
+    // [0, 8) for piece q, so the four lanes of a token read 64 contiguous bytes.
+    // Buffer loads past the chunk's tokens return zeros: without a branch around
+    // them the registers are not copied (and the loads waited for) at a join.
+    uint4 xr[4];
+    auto load_sub = [&](int k, int sub) {
+        const int left = T - k * kChunk;  // <= 0 past the last chunk
+        // uniform values, said so: a descriptor in vector registers would be loaded from lane by lane
+        const int rows = __builtin_amdgcn_readfirstlane(left < 0 ? 0 : (left < kChunk ? left : kChunk));
+        const uint64_t base = reinterpret_cast<uint64_t>(x + (rows ? (long)k * kChunk * kDim : 0));
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)base);
+        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(base >> 32));
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+            reinterpret_cast<void*>((uint64_t)hi << 32 | lo), 0, rows * kDim * 2, 0x00020000);
+        const int off = (sub * kSub + col) * kDim * 2 + 16 * grp;
 #pragma unroll
-    for (int s = 0; s < SPW; ++s) {
-        const int t0 = chunk * kChunk + (wave + kWaves * s) * kSub;
-        if (t0 < T) {
-            const int tok = t0 + col < T ? t0 + col : t0;
-            const uint4* src = reinterpret_cast<const uint4*>(x + (long)tok * kDim + 8 * grp);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) xr[s][q] = src[4 * q];
-        }
-    }
+        for (int q = 0; q < 4; ++q)
+            xr[q] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off + 64 * q, 0, 0));
+    };
+    // the wave's sub-tile in turn u of a chunk
+    auto sub_in = [&](int u) { return sub_of((u * G + g) * JU + (gw >> 2), gw & 3); };
+    load_sub(slot, sub_in(0));
 
-    // centre operand: lane (col, grp) holds centre nb*16 + col at the same
-    // channels, one contiguous 1 KB wave load per piece (operand-order tables)
-    const uint4* ghi = reinterpret_cast<const uint4*>(thi + bh * CP * kDim);
-    const uint4* glo = reinterpret_cast<const uint4*>(tlo + bh * CP * kDim);
-    uint4 bhi[kRegB ? NB : 1][4], blo[kRegB && LO ? NB : 1][4];
-    uint4* sbh = reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(smem) + kWaves * kSub * kXPitch);
-    uint4* sbl = sbh + CP * kDim / 8;
-    if constexpr (kRegB) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                bhi[nb][q] = ghi[(nb * 4 + q) * 64 + lane];
-                if constexpr (LO) blo[nb][q] = glo[(nb * 4 + q) * 64 + lane];
-            }
-    } else {
-        for (int i = tid; i < CP * kDim / 8; i += kThreads) {
-            sbh[i] = ghi[i];
-            if constexpr (LO) sbl[i] = glo[i];
+    // centre operands: lane (col, grp) reads centre nb*16 + col at the same channels,
+    // one contiguous 1 KB wave read per piece (operand-order tables)
+    {
+        const uint4* ghi = reinterpret_cast<const uint4*>(thi + bh * CP * kDim);
+        const uint4* glo = reinterpret_cast<const uint4*>(tlo + bh * CP * kDim);
+        for (int i = tid; i < kTab; i += W::threads) {
+            s_hi[i] = ghi[i];
+            if constexpr (LO)
+                if (!vrule) s_lo[i] = glo[i];
         }
-        __syncthreads();
+        for (int i = tid; i < CP; i += W::threads) s_cnt[i] = 0;
     }
-    auto b_hi = [&](int nb, int q) -> uint4 {
-        if constexpr (kRegB) return bhi[nb][q];
-        else return sbh[(nb * 4 + q) * 64 + lane];
-    };
-    auto b_lo = [&](int nb, int q) -> uint4 {
-        if constexpr (kRegB) return blo[LO ? nb : 0][q];
-        else return sbl[(nb * 4 + q) * 64 + lane];
-    };
     // |c|^2 of the centres nb*16 + 4*grp + r whose distances this lane holds
     float4 cn[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) cn[nb] = *reinterpret_cast<const float4*>(tnorm + bh * CP + nb * 16 + 4 * grp);
+    __syncthreads();
 
-    float4_t sums[NB][8];  // onehot^T X: rows nb*16 + 4*grp + r, channels db*16 + col
-    float4_t cnt[NB];      // onehot^T 1: member counts of rows nb*16 + 4*grp + r
+    // twice the part's sums: clusters 16*(nb0 + b) + 4*grp + r, channels d0 + 16*h + col
+    float4_t part[MB][NH];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        cnt[nb] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+    for (int b = 0; b < MB; ++b)
 #pragma unroll
-        for (int db = 0; db < 8; ++db) sums[nb][db] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    const half4_t ones = (half4_t){(_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f};
-    // transpose reads: lane i of 16-lane row g points at token 4g + i/4, channel
-    // 16*db + 4*(i%4) and receives tokens 4g + r, channel 16*db + i (r = 0..3)
-    const uint16_t* xt = xs + (4 * grp + (col >> 2)) * kXPitch + 4 * (col & 3);
+        for (int h = 0; h < NH; ++h) part[b][h] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+    const int nb0 = MB * (gw >> 2), d0 = 32 * (gw & 3);
+    const uint32_t mine0 = (uint32_t)(16 * nb0 + col) * 0x01010101u;
+    // transpose reads: lane i of 16-lane row r points at token 4r + i/4, channel
+    // d0 + 4*(i%4) and receives tokens 4r + (0..3), channel d0 + i
+    const uint16_t* xt = s_x + (4 * grp + (col >> 2)) * kXPitch + d0 + 4 * (col & 3);
 
+    // ids of the wave's sub-tile at t0 (token rows in xr), staged with its rows
+    auto assign_sub = [&](int t0, int k_next, int sub_next) {
+        const bool live = t0 + col < T;
+        if (psum != nullptr) {
+            // rows past T are zeros, so that they add nothing
+            uint4* row = reinterpret_cast<uint4*>(s_x + (gw * kSub + col) * kXPitch + 8 * grp);
 #pragma unroll
-    for (int s = 0; s < SPW; ++s) {
-        const int t0 = chunk * kChunk + (wave + kWaves * s) * kSub;
-        if (t0 >= T) break;
+            for (int q = 0; q < 4; ++q) row[4 * q] = xr[q];
+        }
         // S^T = C X^T: lane (col, grp) gets <c, x> for token t0 + col and
         // centres nb*16 + 4*grp + r
         float4_t acc[NB];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            acc[nb] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+        for (int nb = 0; nb < NB; ++nb) acc[nb] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+        if (LO && !vrule) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(b_hi(nb, q)), as_h8(xr[s][q]), acc[nb], 0, 0, 0);
-                if constexpr (LO)
-                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(b_lo(nb, q)), as_h8(xr[s][q]), acc[nb], 0, 0, 0);
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) {
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(s_hi[(nb * 4 + q) * 64 + lane]), as_h8(xr[q]), acc[nb], 0, 0, 0);
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(s_lo[LO ? (nb * 4 + q) * 64 + lane : 0]), as_h8(xr[q]), acc[nb], 0, 0, 0);
+                }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_h8(s_hi[(nb * 4 + q) * 64 + lane]), as_h8(xr[q]), acc[nb], 0, 0, 0);
+        }
+        float xn = 0.0f;
+        if (vrule) {
+            if (xn_row != nullptr && !xnorm_new) {
+                xn = xn_row[min(t0 + col, T - 1)];
+            } else {
+                xn = token_half_norm(xr);
+                if (xn_row != nullptr && grp == 0 && live) xn_row[t0 + col] = xn;
             }
         }
-        int bi;
+        load_sub(k_next, sub_next);  // the rows are staged and multiplied: their registers take the next ones
+        int bi;  // index less 4 * grp within the lane's scan
         if (!vrule) {
             // K: nearest of this lane's centres, scanned in increasing index
             // order (a strict < keeps the lower index on ties), then across the
             // four row groups holding the same token
             float bd = fmaf(-2.0f, acc[0][0], cn[0].x);
-            bi = 4 * grp;
+            bi = 0;
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -360,11 +417,11 @@ kmeans_assign_kernel(
                     const float d = fmaf(-2.0f, acc[nb][r], cnorm(cn[nb], r));
                     const bool take = d < bd;
                     bd = take ? d : bd;
-                    bi = take ? nb * 16 + 4 * grp + r : bi;
+                    bi = take ? nb * 16 + r : bi;
                 }
+            bi += 4 * grp;
             token_argmin(bd, bi);
         } else {
-            const float xn = token_half_norm(xr[s]);
             if (vgroup) {
                 // decode groups: fp32(fp16(|x|^2 + |c|^2) - 2 <x, c>), lowest index on ties
                 float bd = INFINITY;
@@ -377,8 +434,9 @@ kmeans_assign_kernel(
                         const float d = fmaf(-2.0f, acc[nb][r], e);
                         const bool take = d < bd;
                         bd = take ? d : bd;
-                        bi = take ? nb * 16 + 4 * grp + r : bi;
+                        bi = take ? nb * 16 + r : bi;
                     }
+                bi += 4 * grp;
                 token_argmin(bd, bi);
             } else {
                 // Lloyd: fp16 cdist.  The winner is the lowest index whose fp16
@@ -397,102 +455,143 @@ kmeans_assign_kernel(
                         dmin = fminf(dmin, d16[nb][r]);
                     }
                 dmin = token_min(dmin);
-                const float thr = root_bound_sq(dmin);
+                // the largest fp32 value below M^2 (dmin itself when it is infinite)
+                const float most = dmin == INFINITY ? dmin : i2f(f2i(root_bound_sq(dmin)) - 1);
                 bi = 1 << 20;
 #pragma unroll
                 for (int nb = NB - 1; nb >= 0; --nb)
 #pragma unroll
                     for (int r = 3; r >= 0; --r)
-                        if (d16[nb][r] < thr || d16[nb][r] == dmin) bi = nb * 16 + 4 * grp + r;
-                bi = token_min_index(bi);
+                        if (d16[nb][r] <= most) bi = nb * 16 + r;
+                bi = token_min_index(bi + 4 * grp);
             }
         }
         // every lane of column col now holds the id of token t0 + col
-        if (grp == 0 && t0 + col < T) ids[t0 + col] = bi;
-        if (psum != nullptr) {
-            // stage the tile: lane (col, grp) writes token col's channels 32 q + 8 grp + [0, 8)
-            uint4* row = reinterpret_cast<uint4*>(xs + col * kXPitch + 8 * grp);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) row[4 * q] = xr[s][q];
-            // A = onehot^T: lane (col, grp) holds [cluster nb*16 + col][tokens 4*grp + i],
-            // the tokens' ids fetched from the lanes of row 0 that hold them
-            int tid4[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) tid4[i] = __builtin_amdgcn_ds_bpermute((4 * grp + i) * 4, bi);
-            half4_t oh[NB];
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const bool in = (t0 + 4 * grp + i < T) && tid4[i] == nb * 16 + col;
-                    oh[nb][i] = in ? (_Float16)1.0f : (_Float16)0.0f;
-                }
-            }
-            wave_sync();
-#pragma unroll
-            for (int db = 0; db < 8; ++db) {
-                const half4_t xb = __builtin_bit_cast(
-                    half4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(xt + 16 * db)));
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-                    sums[nb][db] = __builtin_amdgcn_mfma_f32_16x16x16f16(oh[nb], xb, sums[nb][db], 0, 0, 0);
-            }
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) cnt[nb] = __builtin_amdgcn_mfma_f32_16x16x16f16(oh[nb], ones, cnt[nb], 0, 0, 0);
-            wave_sync();  // tile reads done before the next tile is staged
+        if (grp == 0 && live) ids[t0 + col] = bi;
+        if (psum == nullptr) return;
+        if (grp == 0) {
+            // tokens 4r..4r+3 of all of the unit's sub-tiles are contiguous
+            g_id[(col >> 2) * (4 * US) + 4 * gw + (col & 3)] = (uint8_t)(live ? bi & (kMaxClusters - 1) : 0);
+            if (live && bi < CP) atomicAdd(&s_cnt[bi], 1);
         }
-    }
-    if (psum == nullptr) return;
-    // waves 4..7 write regions 0..3 (the regions reuse the tiles' LDS), waves
-    // 0..3 add theirs, then the regions are added in order: a fixed association
-    __syncthreads();
-    float* reg = reinterpret_cast<float*>(smem) + (wave & (kRegions - 1)) * region_floats<NB>();
-    auto region_pass = [&](bool add) {
+    };
+    // r_j of the unit's jj-th j for this wave's centres and channels
+    auto unit_sum = [&](int jj, float4_t (&r)[MB][NH]) {
+        const uint4 i4 = *reinterpret_cast<const uint4*>(g_id + grp * (4 * US) + 16 * jj);
+        const uint32_t id4[4] = {i4.x, i4.y, i4.z, i4.w};
+        float4_t S[2][MB][NH];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
+        for (int e = 0; e < 4; ++e) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float* dst = reg + (nb * 16 + 4 * grp + r) * kRPitch;
+            for (int b = 0; b < MB; ++b)
 #pragma unroll
-                for (int db = 0; db < 8; ++db) dst[db * 16 + col] = (add ? dst[db * 16 + col] : 0.0f) + sums[nb][db][r];
-                if (col == 0) dst[kDim] = (add ? dst[kDim] : 0.0f) + cnt[nb][r];
+                for (int h = 0; h < NH; ++h)
+                    if ((e & 1) == 0) S[e >> 1][b][h] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+            half4_t xb[NH];
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+                xb[h] = __builtin_bit_cast(half4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                        (lds_short4_t*)(xt + (4 * jj + e) * kSub * kXPitch + 16 * h)));
+#pragma unroll
+            for (int b = 0; b < MB; ++b) {
+                const half4_t oh = one_hot4(id4[e], mine0 + b * 0x10101010u);
+#pragma unroll
+                for (int h = 0; h < NH; ++h)
+                    S[e >> 1][b][h] = __builtin_amdgcn_mfma_f32_16x16x16f16(oh, xb[h], S[e >> 1][b][h], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                r[b][h] = S[0][b][h] + S[1][b][h];
+                asm volatile("" : "+v"(r[b][h]));  // summed here: the S are not held on
             }
     };
-    if (wave >= kRegions) region_pass(false);
-    __syncthreads();
-    if (wave < kRegions) region_pass(true);
-    __syncthreads();
-    const float* r0 = reinterpret_cast<const float*>(smem);
-    float* ps = psum + ((bh * chunks) + chunk) * (long)C * kDim;
-    for (int i = tid; i < C * kDim / 4; i += kThreads) {
-        const int o = (i >> 5) * kRPitch + (i & 31) * 4;
-        float4 s = *reinterpret_cast<const float4*>(r0 + o);
+
+    for (int k = slot; k < chunks; k += slots) {
+        float4_t tot[MB][NH];
 #pragma unroll
-        for (int w = 1; w < kRegions; ++w) {
-            const float4 v = *reinterpret_cast<const float4*>(r0 + w * region_floats<NB>() + o);
-            s.x += v.x;
-            s.y += v.y;
-            s.z += v.z;
-            s.w += v.w;
+        for (int u = 0; u < W::turns; ++u) {
+            assign_sub(k * kChunk + sub_in(u) * kSub, u + 1 < W::turns ? k : k + slots, sub_in((u + 1) % W::turns));
+            if (psum == nullptr) continue;
+            __syncthreads();  // the unit's rows and ids are staged
+#pragma unroll
+            for (int jj = 0; jj < JU; ++jj) {
+                float4_t r[MB][NH];
+                unit_sum(jj, r);
+                if constexpr (G > 1) {
+#pragma unroll
+                    for (int b = 0; b < MB; ++b)
+#pragma unroll
+                        for (int h = 0; h < NH; ++h) tot[b][h] = r[b][h];
+                } else {
+#pragma unroll
+                    for (int b = 0; b < MB; ++b)
+#pragma unroll
+                        for (int h = 0; h < NH; ++h) tot[b][h] = u == 0 && jj == 0 ? r[b][h] : tot[b][h] + r[b][h];
+                }
+            }
+            __syncthreads();  // the rows are read before the next unit (or the sums) overwrite them
         }
-        *reinterpret_cast<float4*>(ps + (long)i * 4) = s;
-    }
-    if (tid < C) {
-        float n = r0[tid * kRPitch + kDim];
+        if constexpr (G == 1) {
+            if (psum != nullptr) {
 #pragma unroll
-        for (int w = 1; w < kRegions; ++w) n += r0[w * region_floats<NB>() + tid * kRPitch + kDim];
-        pcnt[(bh * chunks + chunk) * C + tid] = (int)n;
+                for (int b = 0; b < MB; ++b)
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) part[b][h] += tot[b][h];
+            }
+        } else {
+            // one chunk per workgroup: ((r_0 + r_1) + r_2) + r_3 by group 0
+            if (psum == nullptr) return;
+            float* sums = reinterpret_cast<float*>(s_rows);  // every group's r_j but group 0's
+            auto at = [&](int j, int b, int h, int r) -> float& {
+                return sums[(j - 1) * kSumFloats + (16 * (nb0 + b) + 4 * grp + r) * kDim + d0 + 16 * h + col];
+            };
+            if (g > 0) {
+#pragma unroll
+                for (int b = 0; b < MB; ++b)
+#pragma unroll
+                    for (int h = 0; h < NH; ++h)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) at(g, b, h, r) = tot[b][h][r];
+            }
+            __syncthreads();
+            if (g == 0) {
+#pragma unroll
+                for (int b = 0; b < MB; ++b)
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) {
+#pragma unroll
+                        for (int j = 1; j < 4; ++j)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) tot[b][h][r] += at(j, b, h, r);
+                        part[b][h] += tot[b][h];
+                    }
+            }
+        }
     }
+    if (psum == nullptr || g > 0) return;
+    float* ps = psum + ((bh * slots) + slot) * (long)C * kDim + d0 + col;
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int c = 16 * (nb0 + b) + 4 * grp + r;
+            if (c >= C) continue;
+#pragma unroll
+            for (int h = 0; h < NH; ++h) ps[(long)c * kDim + 16 * h] = 0.5f * part[b][h][r];
+        }
+    for (int i = tid; i < C; i += W::GW * kWave) pcnt[(bh * slots + slot) * C + i] = s_cnt[i];
 }
 
 // One workgroup (512 threads: channel x chunk residue mod 4) per (cluster,
 // problem); the four parts of the chunk sum meet in LDS and are added in a
 // fixed order.  Writes the centre, then either its tables for the next
 // assignment (thi non-null) or the fp16 result (thi null).
-constexpr int kParts = 4;
 __global__ void __launch_bounds__(kParts * kDim) kmeans_update_kernel(
     Problems P, float* __restrict__ centers, const float* __restrict__ psum, const int* __restrict__ pcnt, int C,
-    int Cp, int chunks, uint16_t* __restrict__ thi, uint16_t* __restrict__ tlo, float* __restrict__ tnorm) {
+    int Cp, int slots, uint16_t* __restrict__ thi, uint16_t* __restrict__ tlo, float* __restrict__ tnorm) {
     __shared__ float s_part[kParts][kDim];
     __shared__ int s_n[kParts];
     __shared__ float s_w[2];
@@ -501,10 +600,10 @@ __global__ void __launch_bounds__(kParts * kDim) kmeans_update_kernel(
     const int d = threadIdx.x & (kDim - 1), par = threadIdx.x >> 7;
     float s = 0.0f;
     int n = 0;
-    const float* src = psum + (bh * chunks) * (long)C * kDim + c * kDim + d;
-    const int* cnt = pcnt + bh * chunks * C + c;
+    const float* src = psum + (bh * slots) * (long)C * kDim + c * kDim + d;
+    const int* cnt = pcnt + bh * slots * C + c;
 #pragma unroll 16
-    for (int k = par; k < chunks; k += kParts) {
+    for (int k = par; k < slots; k += kParts) {
         s += src[(long)k * C * kDim];
         n += cnt[k * C];
     }
@@ -536,13 +635,25 @@ __global__ void __launch_bounds__(kParts * kDim) kmeans_update_kernel(
 // Workspace: fp32 centres, the fp16 hi/lo tables and norms, chunk partials;
 // every array starts on a 256-byte boundary.
 struct Layout {
-    int Cp, chunks;
-    int64_t centers, thi, tlo, tnorm, psum, pcnt, total;
+    int Cp, chunks, slots;
+    int64_t centers, thi, tlo, tnorm, xnorm, psum, pcnt, total;
 };
+// Workgroups per problem of the assignment: one per part (each streams its chunks
+// and writes one partial) once that fills the chip, else one per chunk.  Up to 32
+// centres a part's workgroup has four waves, and two of them per CU are needed (64
+// problems of 8192 tokens, 10 iterations: 543 us by parts, 485 by chunks; 128
+// problems: 832 against 1025); above 32 it has eight and spares twice the partials
+// (C = 64: 32 problems 551 against 447 us, 48 problems 587 against 604, 64
+// problems 620 against 765).
+int slots_for(int BH, int chunks, int Cp) {
+    const int64_t groups = (int64_t)BH * kParts;
+    return chunks > kParts && groups >= (Cp <= 32 ? 2 * kCUs : kCUs * 3 / 4) ? kParts : chunks;
+}
 Layout layout(int BH, int T, int C) {
     Layout L;
     L.Cp = (C + 15) / 16 * 16;
     L.chunks = (T + kChunk - 1) / kChunk;
+    L.slots = slots_for(BH, L.chunks, L.Cp);
     int64_t off = 0;
     auto take = [&](int64_t bytes) {
         const int64_t at = off;
@@ -553,8 +664,9 @@ Layout layout(int BH, int T, int C) {
     L.thi = take((int64_t)BH * L.Cp * kDim * 2);
     L.tlo = take((int64_t)BH * L.Cp * kDim * 2);
     L.tnorm = take((int64_t)BH * L.Cp * 4);
-    L.psum = take((int64_t)BH * L.chunks * C * kDim * 4);
-    L.pcnt = take((int64_t)BH * L.chunks * C * 4);
+    L.xnorm = take((int64_t)BH * T * 4);
+    L.psum = take((int64_t)BH * L.slots * C * kDim * 4);
+    L.pcnt = take((int64_t)BH * L.slots * C * 4);
     L.total = off;
     return L;
 }
@@ -565,33 +677,37 @@ struct Tables {
     float* norm;
 };
 
-template <int NB, bool REGB>
-void launch_nb(bool lo, dim3 grid, hipStream_t st, const Problems& P, const Tables& tb, float* psum, int* pcnt, int T,
-               int C, int chunks) {
+template <int NB, int G>
+void launch_nb(bool lo, dim3 grid, hipStream_t st, const Problems& P, const Tables& tb, float* psum, int* pcnt,
+               float* xnorm, int xnorm_new, int T, int C, int chunks) {
+    const dim3 threads(Split<NB, G>::threads);
     if (lo)
-        hipLaunchKernelGGL((kmeans_assign_kernel<NB, true, REGB>), grid, dim3(kThreads), 0, st, P, tb.hi, tb.lo,
-                           tb.norm, psum, pcnt, T, C, chunks);
+        hipLaunchKernelGGL((kmeans_assign_kernel<NB, true, G>), grid, threads, 0, st, P, tb.hi, tb.lo, tb.norm, psum,
+                           pcnt, xnorm, xnorm_new, T, C, chunks);
     else
-        hipLaunchKernelGGL((kmeans_assign_kernel<NB, false, REGB>), grid, dim3(kThreads), 0, st, P, tb.hi, tb.lo,
-                           tb.norm, psum, pcnt, T, C, chunks);
+        hipLaunchKernelGGL((kmeans_assign_kernel<NB, false, G>), grid, threads, 0, st, P, tb.hi, tb.lo, tb.norm, psum,
+                           pcnt, xnorm, xnorm_new, T, C, chunks);
 }
 
-int launch_assign(const Problems& P, const Tables& tb, float* psum, int* pcnt, int BH, int T, int C, const Layout& L,
-                  hipStream_t st) {
-    const dim3 grid(L.chunks, BH);
+int launch_assign(const Problems& P, const Tables& tb, float* psum, int* pcnt, float* xnorm, int xnorm_new, int BH,
+                  int T, int C, const Layout& L, hipStream_t st) {
+    const dim3 grid(L.slots, BH);
     const bool lo = P.vfrom > 0;
-    const bool regb = (int64_t)L.chunks * BH <= kCUs;  // one workgroup per CU: registers; more: LDS operands
+    // a chunk's sub-tiles over 16 waves instead of four turns of four while the
+    // grid leaves CUs idle (C = 32, 10 iterations: 64 workgroups 117 against 131 us,
+    // 256 134 against 149, 384 192 against 165)
+    const bool wide = L.slots == L.chunks && (int64_t)L.chunks * BH <= kCUs;
     switch (L.Cp / 16) {
     case 1:
-        if (regb) launch_nb<1, true>(lo, grid, st, P, tb, psum, pcnt, T, C, L.chunks);
-        else launch_nb<1, false>(lo, grid, st, P, tb, psum, pcnt, T, C, L.chunks);
+        if (wide) launch_nb<1, 4>(lo, grid, st, P, tb, psum, pcnt, xnorm, xnorm_new, T, C, L.chunks);
+        else launch_nb<1, 1>(lo, grid, st, P, tb, psum, pcnt, xnorm, xnorm_new, T, C, L.chunks);
         break;
     case 2:
-        if (regb) launch_nb<2, true>(lo, grid, st, P, tb, psum, pcnt, T, C, L.chunks);
-        else launch_nb<2, false>(lo, grid, st, P, tb, psum, pcnt, T, C, L.chunks);
+        if (wide) launch_nb<2, 4>(lo, grid, st, P, tb, psum, pcnt, xnorm, xnorm_new, T, C, L.chunks);
+        else launch_nb<2, 1>(lo, grid, st, P, tb, psum, pcnt, xnorm, xnorm_new, T, C, L.chunks);
         break;
-    case 3: launch_nb<3, false>(lo, grid, st, P, tb, psum, pcnt, T, C, L.chunks); break;
-    default: launch_nb<4, false>(lo, grid, st, P, tb, psum, pcnt, T, C, L.chunks); break;
+    case 3: launch_nb<3, 1>(lo, grid, st, P, tb, psum, pcnt, xnorm, xnorm_new, T, C, L.chunks); break;
+    default: launch_nb<4, 1>(lo, grid, st, P, tb, psum, pcnt, xnorm, xnorm_new, T, C, L.chunks); break;
     }
     return reskv_host::check_launch("kmeans_assign_kernel");
 }
@@ -657,11 +773,12 @@ int run_kmeans(const Problems& P, const float* const init[2], int BH, int T, int
         }
         if (launch_prep(centers, tb, BH, C, L.Cp, P.vfrom, st)) return 1;
     }
+    float* xnorm = (float*)(w + L.xnorm);
     for (int it = 0; it < iterations; ++it) {
-        if (launch_assign(P, tb, psum, pcnt, BH, T, C, L, st)) return 1;
+        if (launch_assign(P, tb, psum, pcnt, xnorm, it == 0, BH, T, C, L, st)) return 1;
         const bool last = it == iterations - 1;
         hipLaunchKernelGGL(kmeans_update_kernel, dim3(C, BH), dim3(kParts * kDim), 0, st, P, centers, psum, pcnt, C,
-                           L.Cp, L.chunks, last ? nullptr : tb.hi, tb.lo, tb.norm);
+                           L.Cp, L.slots, last ? nullptr : tb.hi, tb.lo, tb.norm);
         if (reskv_host::check_launch("kmeans_update_kernel")) return 1;
     }
     return 0;
@@ -689,7 +806,7 @@ extern "C" int reskv_kmeans_assign(const void* x, const float* centers, int32_t*
     const Problems P{{(const uint16_t*)x, (const uint16_t*)x}, {ids, ids}, {nullptr, nullptr}, BH, vfrom, 1};
     hipStream_t st = (hipStream_t)stream;
     if (launch_prep(centers, tb, BH, C, L.Cp, vfrom, st)) return 1;
-    return launch_assign(P, tb, nullptr, nullptr, BH, T, C, L, st);
+    return launch_assign(P, tb, nullptr, nullptr, nullptr, 0, BH, T, C, L, st);
 }
 
 extern "C" int reskv_linspace_rows(int T, int C, int32_t* rows) {
