@@ -45,6 +45,21 @@ int reskv_llama_qkv_rope(const void* qkv, const float* cos, const float* sin, co
                          void* cache_raw, void* cache_v, const int64_t* slot, int64_t stride_b,
                          int64_t stride_h, int64_t stride_t, void* stream);
 
+/* The prompt's counterpart of qkv_rope: qkv fp16 [B, T, (Hq + 2 Hk) * 128]; cos/sin
+ * fp32 [T, 64], row t for token t, same rotation and rounding.  Writes qr fp16
+ * [B, Hq, T, 128] (rotated Q), k and kr [B, Hk, T, 128] (raw and rotated K) and v
+ * [B, Hk, T, 128].  Everything contiguous and 16-byte aligned. */
+int reskv_llama_prefill_split(const void* qkv, const float* cos, const float* sin, int B, int T, int Hq, int Hk,
+                              void* qr, void* k, void* kr, void* v, void* stream);
+
+/* Causal attention over a prompt: q fp16 [B, Hq, T, 128] and k [B, Hk, T, 128]
+ * (both rotated), v [B, Hk, T, 128], out [B, T, Hq, 128], contiguous and 16-byte
+ * aligned; Hq / Hk 1, 2 or a multiple of 4; scaling > 0.  Scores and softmax in
+ * fp32; the softmax weights are rounded to fp16 for the product with V, which
+ * accumulates in fp32. */
+int reskv_llama_prefill_attention(const void* q, const void* k, const void* v, void* out, int B, int Hq, int Hk,
+                                  int T, float scaling, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

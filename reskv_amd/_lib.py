@@ -14,7 +14,7 @@ LIB_PATH = _HERE / "libreskv_hip.so"
 _vp, _i, _i64, _f = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
 
 # reskv_abi_version() of the library these signatures describe
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 
 class CTensor(ctypes.Structure):
@@ -70,6 +70,8 @@ SIGNATURES = {
     # include/reskv_llama.h: fused steps of the end-to-end decode harness
     "reskv_llama_rmsnorm": (_i, [_vp, _vp, _vp, _i, _i, _f, _vp]),
     "reskv_llama_silu_mul": (_i, [_vp, _vp, _i, _i, _vp]),
+    "reskv_llama_prefill_split": (_i, [_vp] * 3 + [_i] * 4 + [_vp] * 5),
+    "reskv_llama_prefill_attention": (_i, [_vp] * 4 + [_i] * 4 + [_f, _vp]),
     "reskv_llama_qkv_rope": (_i, [_vp] * 4 + [_i, _i, _i] + [_vp] * 9 + [_i64, _i64, _i64, _vp]),
 }
 

@@ -157,6 +157,43 @@ def fused_qkv_rope(qkv, cos, sin, pos, q, qr, k, kr, v, targets=None):
         _stream(qkv)), "reskv_llama_qkv_rope")
 
 
+def fused_prefill_split(qkv, cos, sin, batch, heads, kv_heads):
+    """A prompt's (rotated Q [B, Hq, T, 128], K, rotated K, V [B, Hk, T, 128]) from its fused
+    projection qkv [B * T, (Hq + 2 Hk) * 128]: ``_rotate`` at positions 0 .. T - 1, one launch."""
+    _fp16_rows("qkv", qkv, None, (heads + 2 * kv_heads) * 128)
+    _need(batch > 0 and qkv.shape[0] % batch == 0, "qkv rows must be a multiple of the batch")
+    t = qkv.shape[0] // batch
+    _need(all(x.dtype == torch.float32 and tuple(x.shape) == (t, 64) and x.is_contiguous() for x in (cos, sin)),
+          "cos and sin must be contiguous fp32 tables [T, 64]")
+    _on_gpu(qkv, cos, sin)
+    new = lambda h: torch.empty(batch, h, t, 128, dtype=torch.float16, device=qkv.device)  # noqa: E731
+    qr, k, kr, v = new(heads), new(kv_heads), new(kv_heads), new(kv_heads)
+    _lib.check(_lib.lib().reskv_llama_prefill_split(
+        qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), batch, t, heads, kv_heads, qr.data_ptr(), k.data_ptr(),
+        kr.data_ptr(), v.data_ptr(), _stream(qkv)), "reskv_llama_prefill_split")
+    return qr, k, kr, v
+
+
+def fused_prefill_attention(q, k, v, scaling):
+    """Causal attention of a prompt: q fp16 [B, Hq, T, 128], k and v [B, Hk, T, 128] (q and k
+    rotated), contiguous; returns fp16 [B, T, Hq, 128], one launch."""
+    _need(q.dim() == 4 and k.dim() == 4 and q.shape[3] == 128 and k.shape == v.shape
+          and (q.shape[0], *q.shape[2:]) == (k.shape[0], *k.shape[2:]), "q [B, Hq, T, 128] and k, v [B, Hk, T, 128]")
+    _need(all(x.dtype == torch.float16 and x.is_contiguous() for x in (q, k, v)), "q, k and v must be contiguous fp16")
+    b, hq, t, _ = q.shape
+    _need(_prefill_ratio(hq, k.shape[1]), "the query/KV head ratio must be 1, 2 or a multiple of 4")
+    _on_gpu(q, k, v)
+    out = torch.empty(b, t, hq, 128, dtype=torch.float16, device=q.device)
+    _lib.check(_lib.lib().reskv_llama_prefill_attention(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, hq, k.shape[1], t, float(scaling), _stream(q)),
+        "reskv_llama_prefill_attention")
+    return out
+
+
+def _prefill_ratio(heads, kv_heads):
+    return heads % kv_heads == 0 and (heads // kv_heads in (1, 2) or heads // kv_heads % 4 == 0)
+
+
 def _rotate(x, cos, sin):
     """Rotate-half RoPE in fp32; x [..., 128], cos/sin broadcastable to [..., 64]."""
     xf = x.float()
@@ -215,19 +252,51 @@ class RandomLlama:
             act.mul_(gu[:, s.ffn:])
             flat[r0: r0 + rows] += F.linear(act, p["wd"])
 
+    def _fused(self, t):
+        """Whether the library's kernels take this model's prompts (else torch formulas)."""
+        s = self.shape
+        return (self.device.type == "cuda" and s.head_dim == 128 and _prefill_ratio(s.heads, s.kv_heads)
+                and s.hidden % 8 == 0 and s.hidden <= 8192 and s.ffn % 8 == 0 and t <= 1 << 22)
+
+    def _layer_fused(self, li, p, x, cos, sin, sink, rows=16384):
+        """One layer of the prompt in place on x [B, T, hidden]: the norms, the split and
+        rotation, attention and the activation are single launches, and the residual adds
+        ride in the projections (one rounding of x + y)."""
+        s = self.shape
+        b, t, _ = x.shape
+        flat = x.view(b * t, s.hidden)
+        h = fused_rmsnorm(flat, p["n1"], s.rms_eps, torch.empty_like(flat))
+        qr, k, kr, v = fused_prefill_split(F.linear(h, p["wqkv"]), cos, sin, b, s.heads, s.kv_heads)
+        sink(li, k, kr, v)
+        attn = fused_prefill_attention(qr, kr, v, self.scaling)
+        del qr, k, kr, v
+        flat.addmm_(attn.view(b * t, s.hidden), p["wo"].t())
+        del attn
+        for r0 in range(0, b * t, rows):
+            part = flat[r0: r0 + rows]
+            gu = F.linear(fused_rmsnorm(part, p["n2"], s.rms_eps, h[r0: r0 + rows]), p["wgu"])
+            act = torch.empty(gu.shape[0], s.ffn, dtype=torch.float16, device=x.device)
+            part.addmm_(fused_silu_mul(gu, act), p["wd"].t())
+
     @torch.no_grad()
     def prefill(self, ids, sink, q_rows=2048, logits=False):
         """Causal forward of the prompt ids [B, T]; ``sink(layer, raw_k, rot_k, v)``
         receives each layer's keys and values as [B, Hk, T, 128].  Returns the
         greedy next token per sequence [B] (or, with ``logits``, the last
-        position's logits [B, vocab])."""
+        position's logits [B, vocab]).  On a GPU the layers run through the
+        library's prompt kernels; elsewhere as torch formulas, q_rows queries at
+        a time."""
         s = self.shape
         b, t = ids.shape
         cos, sin = self.rope_tables(t)
         x = self.embed[ids]  # [B, T, hidden]
+        fused = self._fused(t)
         rep = s.heads // s.kv_heads
-        causal = torch.ones(q_rows, t, dtype=torch.bool, device=self.device)
+        causal = None if fused else torch.ones(q_rows, t, dtype=torch.bool, device=self.device)
         for li, p in enumerate(self.layers):
+            if fused:
+                self._layer_fused(li, p, x, cos, sin, sink)
+                continue
             h = _rmsnorm(x, p["n1"], s.rms_eps)
             q, k, v = self._split(F.linear(h, p["wqkv"]))
             del h
