@@ -71,16 +71,16 @@ __device__ __forceinline__ int operand_slot_half(int c, int d) {
     return (((c >> 4) * 4 + (d >> 5)) * 64 + ((d >> 3) & 3) * 16 + (c & 15)) * 8 + (d & 7);
 }
 
-// Centre c of one problem's tables from the fp32 centre v held by threads
-// 0..127 (channel = thread).  Every thread of the workgroup calls it (it holds
-// a barrier); threads >= 128 pass active = false.  K rows carry an fp16 lo
+// Centre c of one problem's tables from the fp32 centre v held by 128 threads
+// (channel = thread % 128; s_w: their two floats of LDS).  Every thread of the
+// workgroup calls it (it holds a barrier); those without a centre pass active = false.  K rows carry an fp16 lo
 // part and the fp32 |c|^2; V rows (fp16 centres) carry the fp16 norm of the
 // reference's cdist, the fp16 sum of fp16-rounded squares.
 __device__ __forceinline__ void store_tables(float v, bool active, bool pad, bool value, int c,
                                              uint16_t* __restrict__ hi, uint16_t* __restrict__ lo,
                                              float* __restrict__ norm, float* s_w) {
 #pragma clang fp contract(off)
-    const int t = threadIdx.x;
+    const int t = threadIdx.x & (kDim - 1);
     if (active) {
         const uint16_t hb = f2h(v);
         const int o = operand_slot_half(c, t);
@@ -91,7 +91,7 @@ __device__ __forceinline__ void store_tables(float v, bool active, bool pad, boo
         if ((t & 63) == 0) s_w[t >> 6] = w;
     }
     __syncthreads();
-    if (t == 0) *norm = pad ? INFINITY : (value ? h2f(f2h(s_w[0] + s_w[1])) : s_w[0] + s_w[1]);
+    if (active && t == 0) *norm = pad ? INFINITY : (value ? h2f(f2h(s_w[0] + s_w[1])) : s_w[0] + s_w[1]);
 }
 
 // Where the problems live: problems [0, split) are rows of tensor 0 and
@@ -585,36 +585,57 @@ kmeans_assign_kernel(
     for (int i = tid; i < C; i += W::GW * kWave) pcnt[(bh * slots + slot) * C + i] = s_cnt[i];
 }
 
-// One workgroup (512 threads: channel x chunk residue mod 4) per (cluster,
-// problem); the four parts of the chunk sum meet in LDS and are added in a
-// fixed order.  Writes the centre, then either its tables for the next
-// assignment (thi non-null) or the fp16 result (thi null).
+// The new centres from the partials: per cluster and channel the sums of the four
+// parts (chunks of equal residue mod 4, in increasing order), added in order.
+// Writes the centre, then either its tables for the next assignment (thi
+// non-null) or the fp16 result (thi null).
+//
+// FEW: at most one partial per part (slots <= 4): 128 threads form a centre from
+// four loads and a workgroup takes kParts centres.  Otherwise a workgroup takes one
+// centre, 128 threads per part, and the parts meet in LDS.  256 problems with 32
+// centres, 4 partials each: 13.5 -> 7 us (8192 workgroups before, 2048 now).
+template <bool FEW>
 __global__ void __launch_bounds__(kParts * kDim) kmeans_update_kernel(
     Problems P, float* __restrict__ centers, const float* __restrict__ psum, const int* __restrict__ pcnt, int C,
     int Cp, int slots, uint16_t* __restrict__ thi, uint16_t* __restrict__ tlo, float* __restrict__ tnorm) {
     __shared__ float s_part[kParts][kDim];
     __shared__ int s_n[kParts];
-    __shared__ float s_w[2];
-    const int c = blockIdx.x;
+    __shared__ float s_w[kParts][2];
+    const int d = threadIdx.x & (kDim - 1), quarter = threadIdx.x >> 7;
+    const int c = FEW ? blockIdx.x * kParts + quarter : blockIdx.x;
     const long bh = blockIdx.y;
-    const int d = threadIdx.x & (kDim - 1), par = threadIdx.x >> 7;
-    float s = 0.0f;
-    int n = 0;
-    const float* src = psum + (bh * slots) * (long)C * kDim + c * kDim + d;
-    const int* cnt = pcnt + bh * slots * C + c;
+    const bool live = c < C;
+    const float* src = psum + (bh * slots) * (long)C * kDim + (live ? c : 0) * kDim + d;
+    const int* cnt = pcnt + bh * slots * C + (live ? c : 0);
+    float s;
+    int n;
+    if constexpr (FEW) {
+        float p[kParts];
+        n = 0;
+#pragma unroll
+        for (int k = 0; k < kParts; ++k) {
+            p[k] = k < slots ? src[(long)k * C * kDim] : 0.0f;
+            n += k < slots ? cnt[k * C] : 0;
+        }
+        s = ((p[0] + p[1]) + p[2]) + p[3];
+    } else {
+        s = 0.0f;
+        n = 0;
 #pragma unroll 16
-    for (int k = par; k < slots; k += kParts) {
-        s += src[(long)k * C * kDim];
-        n += cnt[k * C];
+        for (int k = quarter; k < slots; k += kParts) {
+            s += src[(long)k * C * kDim];
+            n += cnt[k * C];
+        }
+        s_part[quarter][d] = s;
+        if (d == 0) s_n[quarter] = n;
+        __syncthreads();
+        s = ((s_part[0][d] + s_part[1][d]) + s_part[2][d]) + s_part[3][d];
+        n = s_n[0] + s_n[1] + s_n[2] + s_n[3];
     }
-    s_part[par][d] = s;
-    if (d == 0) s_n[par] = n;
-    __syncthreads();
-    s = ((s_part[0][d] + s_part[1][d]) + s_part[2][d]) + s_part[3][d];
-    n = s_n[0] + s_n[1] + s_n[2] + s_n[3];
     const bool value_mode = bh >= P.vfrom;
+    const bool mine = live && (FEW || quarter == 0);
     float nv = 0.0f;
-    if (par == 0) {
+    if (mine) {
         float* cv = centers + (bh * C + c) * kDim + d;
         if (value_mode) {
             nv = n > 0 ? h2f(f2h(s / (float)n)) : 0.0f;  // fp16 centres, empty -> 0
@@ -629,7 +650,7 @@ __global__ void __launch_bounds__(kParts * kDim) kmeans_update_kernel(
     }
     if (thi == nullptr) return;  // uniform over the workgroup
     const long head = bh * Cp * kDim;
-    store_tables(nv, par == 0, false, value_mode, c, thi + head, tlo + head, tnorm + bh * Cp + c, s_w);
+    store_tables(nv, mine, false, value_mode, c, thi + head, tlo + head, tnorm + bh * Cp + c, s_w[FEW ? quarter : 0]);
 }
 
 // Workspace: fp32 centres, the fp16 hi/lo tables and norms, chunk partials;
@@ -777,8 +798,10 @@ int run_kmeans(const Problems& P, const float* const init[2], int BH, int T, int
     for (int it = 0; it < iterations; ++it) {
         if (launch_assign(P, tb, psum, pcnt, xnorm, it == 0, BH, T, C, L, st)) return 1;
         const bool last = it == iterations - 1;
-        hipLaunchKernelGGL(kmeans_update_kernel, dim3(C, BH), dim3(kParts * kDim), 0, st, P, centers, psum, pcnt, C,
-                           L.Cp, L.slots, last ? nullptr : tb.hi, tb.lo, tb.norm);
+        const bool few = L.slots <= kParts;
+        const auto update = few ? kmeans_update_kernel<true> : kmeans_update_kernel<false>;
+        hipLaunchKernelGGL(update, dim3(few ? (C + kParts - 1) / kParts : C, BH), dim3(kParts * kDim), 0, st, P, centers,
+                           psum, pcnt, C, L.Cp, L.slots, last ? nullptr : tb.hi, tb.lo, tb.norm);
         if (reskv_host::check_launch("kmeans_update_kernel")) return 1;
     }
     return 0;
