@@ -39,7 +39,7 @@ def _cache_heads(query, cache):
 
 
 def _recent_window(recent, query, batch, kv_heads):
-    """The dense window as contiguous (q_rot [B*Hq,128], k_rot, v) or None when empty."""
+    """The dense window as contiguous (q_rot, k_rot, v) or None when empty."""
     if recent is None:
         return None
     q_rot, k_rot, v = recent
@@ -48,9 +48,10 @@ def _recent_window(recent, query, batch, kv_heads):
     if (q_rot.shape != query.shape or k_rot.shape != v.shape or k_rot.dim() != 4 or k_rot.shape[3] != 128
             or tuple(k_rot.shape[:2]) != (batch, kv_heads)):
         raise ValueError("recent Q/K/V shapes do not match the compressed cache")
-    if any(t.device != query.device or t.dtype != torch.float16 for t in (q_rot, k_rot, v)):
-        raise ValueError("recent tensors must be FP16 on the query device")
-    return q_rot.reshape(-1, 128).contiguous(), k_rot.contiguous(), v.contiguous()
+    for t in (q_rot, k_rot, v):
+        if t.dtype != torch.float16 or t.device != query.device:
+            raise ValueError("recent tensors must be FP16 on the query device")
+    return q_rot.contiguous(), k_rot.contiguous(), v.contiguous()
 
 
 @torch.no_grad()

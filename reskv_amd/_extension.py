@@ -42,7 +42,7 @@ def _ptr(t):
 
 
 def _stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _dev_check(*tensors, contiguous=True):
@@ -423,24 +423,41 @@ def _decode(Q, kdesc, vdesc, keep, nh_kv, nh, start_pos, pos_q, rope_base, scali
     return [out, m, l] if return_stats else [out]
 
 
+def _described(t):
+    """What a CompressedTensor's native views are to the library, without their
+    addresses: (format, bits, centroids, width, token row stride, centroid row
+    stride, has metadata, has scale).  The views are checked when they are made and
+    are not replaced afterwards, so this is worked out once for each set of them."""
+    known = t.__dict__.get("_layout")
+    if known is not None and known[0] is t._native:
+        return known[1]
+    c, i, p, m, sc = t._native
+    plan = t.plan
+    if plan.bits == 16 and plan.layout == "unstructured":
+        fmt, bits, sc = _lib.FMT_BITMAP, 16, None
+    elif plan.bits == 16:
+        fmt, bits, sc = (_lib.FMT_STRUCT16 if plan.layout == "structured" else _lib.FMT_TILED), 16, None
+    elif plan.layout == "structured":
+        fmt, bits = _lib.FMT_STRUCT_INT4, 4
+    else:
+        fmt, bits, m = _lib.FMT_QUANT, int(plan.bits), None
+    d = _ctensor(c, i, p, m, sc, fmt, bits)
+    t._layout = (t._native, (d.format, d.bits, d.nc, d.width, d.t_stride, d.c_stride, m is not None, sc is not None))
+    return t._layout[1]
+
+
+def _descriptor(t):
+    fmt, bits, nc, width, ts, cs, has_meta, has_scale = _described(t)
+    c, i, p, m, sc = t._native
+    return _lib.CTensor(c.data_ptr(), i.data_ptr(), p.data_ptr(), m.data_ptr() if has_meta else None,
+                        sc.data_ptr() if has_scale else None, nc, fmt, width, bits, ts, cs)
+
+
 def cache_descriptors(cache):
     """C descriptors of a CompressedKV's key and value tensors (the format the
     family ops derive from the plan) and the tensors they point into."""
-    plan = cache.key.plan
-    out, keep = [], []
-    for t in (cache.key, cache.value):
-        c, i, p, m, sc = t._native
-        if plan.bits == 16 and plan.layout == "unstructured":
-            fmt, bits, sc = _lib.FMT_BITMAP, 16, None
-        elif plan.bits == 16:
-            fmt, bits, sc = (_lib.FMT_STRUCT16 if plan.layout == "structured" else _lib.FMT_TILED), 16, None
-        elif plan.layout == "structured":
-            fmt, bits = _lib.FMT_STRUCT_INT4, 4
-        else:
-            fmt, bits, m = _lib.FMT_QUANT, int(plan.bits), None
-        out.append(_ctensor(c, i, p, m, sc, fmt, bits))
-        keep.extend(x for x in (c, i, p, m, sc) if x is not None)
-    return out[0], out[1], tuple(keep)
+    keep = tuple(x for t in (cache.key, cache.value) for x in t._native if x is not None)
+    return _descriptor(cache.key), _descriptor(cache.value), keep
 
 
 def decode_splits(cache, num_q_heads, splits=0, rope_table=True):
@@ -517,31 +534,36 @@ def decode_step(query2d, cache, num_q_heads, *, position, start_position, scalin
     """One decode call over a CompressedKV: fp16 [B*Hq, 128].
 
     query2d fp16 [B*Hq, 128] pre-RoPE, contiguous.  ``recent`` is None or
-    (rotated query fp16 [B*Hq, 128], rotated K and V fp16 [B, Hk, Tr, 128],
+    (rotated query fp16, B*Hq rows of 128, rotated K and V fp16 [B, Hk, Tr, 128],
     contiguous); the split merge then joins the window before it writes the
     output (``reskv_decode_recent``), so a step is two kernel launches.
     """
-    kdesc, vdesc, keep = cache_descriptors(cache)
     dev = query2d.device
-    _dev_check(query2d, *keep, contiguous=False)
+    _require(query2d.is_cuda and cache.key.payload.device == dev and cache.value.payload.device == dev,
+             "all tensors must be on the same GPU")
+    if recent is not None:
+        _dev_check(query2d, *recent)
+    if torch._C._cuda_getDevice() != dev.index:
+        with torch.cuda.device(dev):
+            return decode_step(query2d, cache, num_q_heads, position=position, start_position=start_position,
+                               scaling=scaling, inv_freq=inv_freq, rope_theta=rope_theta, splits=splits,
+                               recent=recent)
     b, kh = cache.key.centroids.shape[:2]
-    nh, t = int(num_q_heads), cache.seq_len
+    nh, t, splits = int(num_q_heads), cache.seq_len, int(splits)
     freq, table = _rope(inv_freq, rope_theta, dev, int(start_position) + t)
     L = _lib.lib()
-    out = _empty((b * nh, 128), torch.float16, dev)
-    ws = _workspace(L.reskv_decode_workspace_bytes(b, nh, kh, t, int(splits)), dev)
-    common = (query2d.data_ptr(), kdesc, vdesc, freq.data_ptr(), table.data_ptr(), b, nh, kh, t,
-              int(start_position), int(position), float(scaling), int(splits))
-    with torch.cuda.device(dev):
-        if recent is None:
-            _lib.check(L.reskv_decode_rope(*common, out.data_ptr(), None, None, ws.data_ptr(), ws.numel(),
-                                           _stream(dev)), "decode")
-        else:
-            q_rot, k_rec, v_rec = recent
-            _dev_check(q_rot, k_rec, v_rec)
-            tr = int(k_rec.shape[2])
-            _lib.check(L.reskv_decode_recent(*common, q_rot.data_ptr(), k_rec.data_ptr(), v_rec.data_ptr(), tr, tr,
-                                             out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(dev)), "decode")
+    out = torch.empty_like(query2d)
+    ws = _workspace(L.reskv_decode_workspace_bytes(b, nh, kh, t, splits), dev)
+    common = (query2d.data_ptr(), _descriptor(cache.key), _descriptor(cache.value), freq.data_ptr(),
+              table.data_ptr(), b, nh, kh, t, int(start_position), int(position), float(scaling), splits)
+    if recent is None:
+        _lib.check(L.reskv_decode_rope(*common, out.data_ptr(), None, None, ws.data_ptr(), ws.numel(), _stream(dev)),
+                   "decode")
+    else:
+        q_rot, k_rec, v_rec = recent
+        tr = k_rec.shape[2]
+        _lib.check(L.reskv_decode_recent(*common, q_rot.data_ptr(), k_rec.data_ptr(), v_rec.data_ptr(), tr, tr,
+                                         out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(dev)), "decode")
     return out
 
 

@@ -1633,12 +1633,38 @@ PartialLds partial_lds(int kf, const DTensor& k, int vf, const DTensor& v, int G
 // none), and at two for 4:16 below 33 (batch, head) rows (its one-deep
 // prefetch leaves short tiles waiting: 4.6% slower at B = 4 with three).
 // Returns 0 on a runtime error.
-int groups_per_cu(const void* fn, size_t shm, int kf, long heads) {
-    if (shm > 65536 &&
-        hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm) != hipSuccess)
+//
+// The runtime's two answers do not change, so each (instance, LDS size, device)
+// asks for them once per process (about 2 us a call otherwise).
+int resident_groups(const void* fn, size_t shm) {
+    struct Known {
+        const void* fn;
+        size_t shm;
+        int dev, n;
+    };
+    static std::mutex lock;
+    static Known known[256];  // instances in use times centroid counts; what does not fit is asked for again
+    static int count = 0;
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    std::lock_guard<std::mutex> hold(lock);
+    for (int i = 0; i < count; ++i)
+        if (known[i].fn == fn && known[i].shm == shm && known[i].dev == dev) return known[i].n;
+    // the limit only ever grows, so that it covers every size that was asked for
+    size_t most = shm;
+    for (int i = 0; i < count; ++i)
+        if (known[i].fn == fn && known[i].dev == dev && known[i].shm > most) most = known[i].shm;
+    if (most > 65536 &&
+        hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most) != hipSuccess)
         return 0;
     int n = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, kThreads, shm) != hipSuccess || n < 1) return 0;
+    if (count < 256) known[count++] = Known{fn, shm, dev, n};
+    return n;
+}
+
+int groups_per_cu(const void* fn, size_t shm, int kf, long heads) {
+    const int n = resident_groups(fn, shm);
     const bool windows = kf == D_BITMAP || kf == D_BITMAP_W || kf == D_TILED || kf == D_TILED_W;
     const int cap = windows || (kf == D_STRUCT16 && heads <= 32) ? 2 : kMaxGroupsPerCU;
     return n < cap ? n : cap;
