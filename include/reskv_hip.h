@@ -270,6 +270,13 @@ int reskv_decode_dense(const void* q, const void* k, const void* v, const float*
                        int pos_q, float scaling, int splits, void* out, float* m, float* l,
                        void* workspace, int64_t workspace_bytes, void* stream);
 
+/* One decode token into a ring of recent tokens: k_rot, k_raw and v hold a
+ * 128-value row (2-byte values) per (batch, head) at the element strides
+ * strides[6] = {batch, head} of each in that order (channel stride 1); they go to
+ * token `slot` of the contiguous [B, H, cap, 128] buffers.  Rows 16-byte aligned. */
+int reskv_ring_append(const void* k_rot, const void* k_raw, const void* v, const int64_t* strides, void* ring_rot,
+                      void* ring_raw, void* ring_v, int B, int H, int cap, int slot, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -567,6 +567,35 @@ def decode_step(query2d, cache, num_q_heads, *, position, start_position, scalin
     return out
 
 
+_RING_STRIDES = ctypes.c_int64 * 6
+
+
+def ring_append(rings, tokens, slot):
+    """Writes one token's rows (three [B, H, 1, 128] tensors) to token ``slot`` of the
+    three contiguous ring buffers [B, H, cap, 128], one launch.  Returns False, having
+    done nothing, for tensors that torch's copies have to take: other shapes, types,
+    devices or alignments, gradients, or a call that is being compiled."""
+    ring = rings[0]
+    if not ring.is_cuda or ring.element_size() != 2 or ring.shape[3] != 128 or torch.compiler.is_compiling():
+        return False
+    dev = ring.device
+    if torch._C._cuda_getDevice() != dev.index:
+        return False
+    b, h, cap, _ = ring.shape
+    strides = []
+    for x in tokens:
+        if x.shape != (b, h, 1, 128) or x.dtype != ring.dtype or x.device != dev or x.requires_grad:
+            return False
+        sb, sh, _, sd = x.stride()
+        if sd != 1 or sb % 8 or sh % 8 or x.data_ptr() % 16:
+            return False
+        strides += (sb, sh)
+    _lib.check(_lib.lib().reskv_ring_append(
+        tokens[0].data_ptr(), tokens[1].data_ptr(), tokens[2].data_ptr(), _RING_STRIDES(*strides),
+        rings[0].data_ptr(), rings[1].data_ptr(), rings[2].data_ptr(), b, h, cap, slot, _stream(dev)), "ring_append")
+    return True
+
+
 def _check_recent_inputs(comp_out, comp_m, comp_l, v_recent, nh_kv, nh):
     """Shape and dtype checks shared by both merge_recent ops
     (reskv/csrc/attention.cu:850-868, cluster_mass.cu:1469-1476); returns (B, Tr)."""

@@ -26,7 +26,7 @@ try:
 except ImportError:  # the kernels and the harness do not need transformers
     _CacheBase = _LayerBase = object
 
-from ._extension import StepDecoder
+from ._extension import StepDecoder, ring_append
 from .compression import _compress_group, compress
 from .config import ResKVKernelConfig
 from .tensors import CompressedKV, CompressedTensor
@@ -170,9 +170,10 @@ class ResKVLayerCache(_LayerBase):
         else:
             if q_len != 1:
                 raise ValueError("ResKV continuation supports one token per step; chunked prefill is unsupported")
-            self.keys[:, :, self.live: self.live + 1].copy_(key_states)
-            self.raw_keys[:, :, self.live: self.live + 1].copy_(raw)
-            self.values[:, :, self.live: self.live + 1].copy_(value_states)
+            if not ring_append((self.keys, self.raw_keys, self.values), (key_states, raw, value_states), self.live):
+                self.keys[:, :, self.live: self.live + 1].copy_(key_states)
+                self.raw_keys[:, :, self.live: self.live + 1].copy_(raw)
+                self.values[:, :, self.live: self.live + 1].copy_(value_states)
             self._take_token()
             return self.keys[:, :, : self.live], self.values[:, :, : self.live]
         self.length += q_len
