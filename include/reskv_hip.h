@@ -165,7 +165,7 @@ int64_t reskv_decode_workspace_bytes(int B, int Hq, int H, int T, int splits);
 
 /* Split count a decode of these tensors makes (splits<=0: automatic, filling
  * the 256 CUs with as many workgroups as the format's kernel keeps resident
- * per CU, at least two 16-token tiles per wave; >0: min(splits, T, 1024)).
+ * per CU, while a wave has about two 16-token tiles; >0: min(splits, T, 1024)).
  * rope_table: non-zero when the call passes a RoPE table.  Returns -1 (and
  * sets reskv_last_error) on bad arguments. */
 int reskv_decode_splits(const reskv_ctensor* k, const reskv_ctensor* v, int rope_table, int B, int Hq, int H, int T,

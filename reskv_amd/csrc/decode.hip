@@ -23,6 +23,7 @@
 
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 
 using namespace reskv;
@@ -70,6 +71,12 @@ template <> struct Traits<D_Q4> { static constexpr int MB = 0, PQ = 1, DEPTH = 2
 template <> struct Traits<D_Q2> { static constexpr int MB = 0, PQ = 1, DEPTH = 2; static constexpr bool SC = true, CENT = true; };
 template <> struct Traits<D_DENSE> { static constexpr int MB = 0, PQ = 4, DEPTH = 1; static constexpr bool SC = false, CENT = false; };
 
+// Tiles that a partial kernel instance prefetches and works on together.
+template <int KF, int VF>
+constexpr int depth_of(int G) {
+    return Traits<KF>::DEPTH == 2 && Traits<VF>::DEPTH == 2 && G <= 4 ? 2 : 1;
+}
+
 struct DTensor {
     const uint16_t* cent;     // fp16 [BH, nc, 128] (null for dense)
     const int8_t* ids;        // [BH, T] (null for dense)
@@ -86,6 +93,7 @@ struct DParams {
     const float* inv_freq;
     const float4* rope;  // [position][16][cos x4, sin x4] table, or null (sin/cos evaluated in-kernel)
     int Hq, H, T, start_pos, pos_q, splits;
+    int tile_q, tile_r;  // 16-token tiles per wave of the sequence's splits, and the remainder
     float qscale;  // scaling * log2(e): scores come out in the log2 domain
     float one;     // 1.0f, opaque to the compiler: fp16 + fp16 sums as one mixed-precision FMA
     int stage_k, stage_v;  // LDS stage bytes per wave for K and V
@@ -667,16 +675,16 @@ decode_partial_kernel(DParams P) {
         h = pr - b * P.H;
     }
     const long bh = (long)b * P.H + h;
-    const int s0 = (int)(((long)split * P.T) / P.splits);
-    const int s1 = (int)(((long)(split + 1) * P.T) / P.splits);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar registers
     const int t = lane & 15, grp = lane >> 4;  // decode: token of the tile, channel group
     const int hj = lane & 3;                     // query head of this lane within a set
     const int stok = 4 * ((lane >> 2) & 3) + (lane >> 4);  // token of this lane's score
-    // this wave's contiguous share of the split
-    const int t0 = s0 + (int)(((long)wave * (s1 - s0)) / kWaves);
-    const int t1 = s0 + (int)(((long)(wave + 1) * (s1 - s0)) / kWaves);
+    // this wave's contiguous share of the sequence, in whole tiles (only the last
+    // tile of the sequence is partial): tile_q of them, one more for the first tile_r waves
+    const int share = split * kWaves + wave;
+    const int t0 = min(P.T, kTile * (share * P.tile_q + min(share, P.tile_r)));
+    const int t1 = min(P.T, kTile * ((share + 1) * P.tile_q + min(share + 1, P.tile_r)));
 
     uint16_t* s_cent = reinterpret_cast<uint16_t*>(smem);  // region 0: fp16 key centroids [nc][kCPitch]
     uint32_t* s_lut = reinterpret_cast<uint32_t*>(smem + P.lut_off);
@@ -699,7 +707,7 @@ decode_partial_kernel(DParams P) {
     // (two for the quantised formats, whose short tiles would otherwise wait
     // on the load latency; one for the others, and for G = 8, whose registers
     // do not allow two).
-    constexpr int kDepth = (KT::DEPTH == 2 && VT::DEPTH == 2 && G <= 4) ? 2 : 1;
+    constexpr int kDepth = depth_of<KF, VF>(G);
     Prefetch<KF> pk[kDepth];
     Prefetch<VF> pv[kDepth];
 #pragma unroll
@@ -723,10 +731,11 @@ decode_partial_kernel(DParams P) {
         s_qtrig[threadIdx.x] = cs;
         s_qtrig[kHalf + threadIdx.x] = sn;
     }
-    if (threadIdx.x < kLutWords) {
+    constexpr bool kRuns = KF == D_BITMAP || KF == D_BITMAP_W || KF == D_TILED || KF == D_TILED_W;
+    if (kRuns && threadIdx.x < kLutWords) {
         const uint32_t i = threadIdx.x;
         s_lut[i] = perm_selector((i >> 1) & 15u, i < 32, (int)(i & 1));
-    } else if (threadIdx.x < kLutWords + kStructLutWords) {
+    } else if (KF == D_STRUCT16 && threadIdx.x >= kLutWords && threadIdx.x < kLutWords + kStructLutWords) {
         const uint32_t i = threadIdx.x - kLutWords;
         s_lut[kLutWords + i] = struct_selector((i >> 1) & 15u, i >> 5, (int)(i & 1));
     }
@@ -1116,7 +1125,9 @@ __device__ __forceinline__ float block_sum_nt(float v, float* red) {
 
 // Chunk-0 operands of the recent join that a kernel may fetch before its
 // other work: the rotated query value of thread tid < 128, and half a K row:
-// thread tid holds token tid % 128, channels 64 (tid / 128) .. +63.
+// thread tid holds token tid % 128, channels 64 (tid / 128) .. +63.  (Holding the
+// V rows as well cost the split merge a workgroup per SIMD: 1 us slower a call at
+// B = 16, nothing gained at B = 1.)
 struct RecentPre {
     uint4 k[kDim / 16];
     float q;
@@ -1466,29 +1477,33 @@ __global__ void __launch_bounds__(kMergeThreads) merge_recent_kernel(
 // ---------------------------------------------------------------------------
 // The automatic split count fills every CU with as many workgroups as the
 // kernel instance keeps resident per CU (two for most formats at their
-// register use, three for the quantised ones); each wave keeps at least two
-// 16-token tiles so that its next tile's loads overlap the current tile's
-// arithmetic.
+// register use, three for the quantised ones), as far as each wave has about two
+// 16-token tiles, so that its next tile's loads overlap the current tile's
+// arithmetic.  Waves take whole tiles: of the counts that give the fullest wave
+// the same number of tiles, the smallest is taken (fewer records to merge), and
+// instances that work on pairs of tiles get an even number.  With shares in
+// tokens instead (960 tokens in 7 splits: 34 a wave) a wave's last tile held a
+// few tokens and cost a whole one.
 constexpr int kCUs = 256;            // compute units of an MI355X
 constexpr int kMaxGroupsPerCU = 4;   // cap of the automatic split target (and of the workspace bound)
 
-int auto_splits(int B, int H, int T, int per_cu) {
-    const long heads = (long)B * H;
-    long s = ((long)per_cu * kCUs + heads - 1) / heads;
-    const long cap = T / (kWaves * 2 * kTile) > 0 ? T / (kWaves * 2 * kTile) : 1;
-    if (s > cap) s = cap;
-    if (s > kMaxSplits) s = kMaxSplits;
+// The most splits that an automatic count can come to.
+int most_splits(int B, int H, int T, int per_cu) {
+    const long heads = (long)B * H, per_wave = kWaves * 2 * kTile;
+    const long s = std::min({((long)per_cu * kCUs + heads - 1) / heads, (T + per_wave - 1) / per_wave, (long)kMaxSplits});
     return (int)(s < 1 ? 1 : s);
 }
 
-// per_cu: workgroups of the kernel instance resident per CU (automatic splits
-// fill every CU that many times over).
-int resolve_splits(int B, int H, int T, int splits, int per_cu) {
+// per_cu: workgroups of the kernel instance resident per CU; depth: tiles it takes at a time.
+int resolve_splits(int B, int H, int T, int splits, int per_cu, int depth) {
     if (splits > 0) {
         int s = splits < T ? splits : T;
         return s < kMaxSplits ? s : kMaxSplits;
     }
-    return auto_splits(B, H, T, per_cu);
+    const long tiles = ((long)T + kTile - 1) / kTile, most = most_splits(B, H, T, per_cu);
+    long n = (tiles + kWaves * most - 1) / (kWaves * most);  // tiles of the fullest wave
+    n = (n + depth - 1) / depth * depth;
+    return (int)((tiles + kWaves * n - 1) / (kWaves * n));
 }
 
 int64_t workspace_for(int B, int Hq, int S) {
@@ -1605,6 +1620,14 @@ const void* partial_kernel(int kf, int vf, int G, bool tab) {
     return nullptr;
 }
 
+// depth_of at run time.
+int tiles_at_once(int kf, int vf, int G) {
+    const bool two = (kf == D_SINT4 || kf == D_Q4 || kf == D_Q2) && (vf == D_SINT4 || vf == D_Q4 || vf == D_Q2);
+    static_assert(depth_of<D_SINT4, D_SINT4>(4) == 2 && depth_of<D_Q4, D_Q2>(4) == 2 && depth_of<D_Q2, D_Q2>(8) == 1 &&
+                  depth_of<D_BITMAP, D_BITMAP>(4) == 1 && depth_of<D_STRUCT16, D_STRUCT16>(4) == 1, "tile pairs");
+    return two && G <= 4 ? 2 : 1;
+}
+
 // LDS layout of one partial workgroup: centroid table (or the cross-wave merge
 // records, whichever is larger), permute tables, per-wave weight and V tiles,
 // per-wave K and V stages.
@@ -1680,7 +1703,7 @@ int splits_for(int kf, const DTensor& k, int vf, const DTensor& v, int G, bool t
         per_cu = groups_per_cu(fn, partial_lds(kf, k, vf, v, G).bytes, kf, (long)B * H);
         RESKV_REQUIRE(per_cu > 0, "decode occupancy query failed: %s", hipGetErrorString(hipGetLastError()));
     }
-    *out = resolve_splits(B, H, T, splits, per_cu);
+    *out = resolve_splits(B, H, T, splits, per_cu, tiles_at_once(kf, vf, G));
     return 0;
 }
 
@@ -1697,13 +1720,13 @@ int run_decode(const void* q, int kf, const DTensor& k, int vf, const DTensor& v
     const void* fn = partial_kernel(kf, vf, G, rope != nullptr);
     RESKV_REQUIRE(fn != nullptr, "K and V residual formats must match (INT4/INT2 may mix)");
     // the smallest split count these sizes can take, checked before any runtime call
-    RESKV_REQUIRE(ws != nullptr && ws_bytes >= workspace_for(B, Hq, resolve_splits(B, H, T, splits, 1)),
+    RESKV_REQUIRE(ws != nullptr && ws_bytes >= workspace_for(B, Hq, resolve_splits(B, H, T, splits, 1, 2)),
                   "decode workspace too small");
     const PartialLds L = partial_lds(kf, k, vf, v, G);
     RESKV_REQUIRE(L.bytes <= 160 * 1024, "decode LDS requirement %zu exceeds 160 KiB", L.bytes);
     const int per_cu = groups_per_cu(fn, L.bytes, kf, (long)B * H);  // also sets the instance's LDS limit
     RESKV_REQUIRE(per_cu > 0, "decode occupancy query failed: %s", hipGetErrorString(hipGetLastError()));
-    const int S = resolve_splits(B, H, T, splits, per_cu);
+    const int S = resolve_splits(B, H, T, splits, per_cu, tiles_at_once(kf, vf, G));
     RESKV_REQUIRE(ws != nullptr && ws_bytes >= workspace_for(B, Hq, S), "decode workspace too small");
     DParams p{};
     p.q = (const uint16_t*)q;
@@ -1718,6 +1741,9 @@ int run_decode(const void* q, int kf, const DTensor& k, int vf, const DTensor& v
     p.start_pos = start_pos;
     p.pos_q = pos_q;
     p.splits = S;
+    const int tiles = (int)(((long)T + kTile - 1) / kTile);
+    p.tile_q = tiles / (S * kWaves);
+    p.tile_r = tiles % (S * kWaves);
     p.qscale = scaling * kLog2e;
     p.one = 1.0f;
     p.stage_k = L.stage_k;
@@ -1751,7 +1777,7 @@ int run_decode(const void* q, int kf, const DTensor& k, int vf, const DTensor& v
 
 extern "C" int64_t reskv_decode_workspace_bytes(int B, int Hq, int H, int T, int splits) {
     if (B <= 0 || Hq <= 0 || H <= 0 || T <= 0) return 0;
-    return workspace_for(B, Hq, resolve_splits(B, H, T, splits, kMaxGroupsPerCU));
+    return workspace_for(B, Hq, splits > 0 ? resolve_splits(B, H, T, splits, 1, 1) : most_splits(B, H, T, kMaxGroupsPerCU));
 }
 
 extern "C" int reskv_decode_splits(const reskv_ctensor* k, const reskv_ctensor* v, int rope_table, int B, int Hq,
@@ -1849,7 +1875,15 @@ extern "C" int reskv_decode_recent_noalloc(const void* q, const reskv_ctensor* k
                                            const void* q_rope, const void* k_recent, const void* v_recent, int Tr,
                                            int r_stride, void* out, void* stream) {
     RESKV_REQUIRE(B > 0 && Hq > 0 && H > 0 && T > 0, "batch, head and token counts must be positive");
-    const int64_t need = reskv_decode_workspace_bytes(B, Hq, H, T, splits);
+    int64_t need = reskv_decode_workspace_bytes(B, Hq, H, T, splits);
+    if (splits <= 0 && need > kNoAllocScratchBytes && T > kWaves * 2 * kTile) {
+        // one split less (whole pairs of tiles per wave) may still fit
+        const int whole = std::min(most_splits(B, H, T, kMaxGroupsPerCU), T / (kWaves * 2 * kTile));
+        if (workspace_for(B, Hq, whole) <= kNoAllocScratchBytes) {
+            splits = whole;
+            need = workspace_for(B, Hq, whole);
+        }
+    }
     RESKV_REQUIRE(need <= kNoAllocScratchBytes,
                   "reskv_decode_recent_noalloc: these sizes need %lld bytes of split-K scratch; the "
                   "allocation-free entry point holds %lld (use reskv_decode_recent with a workspace)",
