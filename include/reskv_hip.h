@@ -277,6 +277,12 @@ int reskv_decode_dense(const void* q, const void* k, const void* v, const float*
 int reskv_ring_append(const void* k_rot, const void* k_raw, const void* v, const int64_t* strides, void* ring_rot,
                       void* ring_raw, void* ring_v, int B, int H, int cap, int slot, void* stream);
 
+/* Range check of two tensors' cluster ids: flags[0] (flags[1]) is set to 1 when one
+ * of the nk k_ids (nv v_ids) lies outside [0, k_count) ([0, v_count)), and is left
+ * alone otherwise (device int32; the caller clears it). */
+int reskv_ids_in_range(const int32_t* k_ids, int64_t nk, int k_count, const int32_t* v_ids, int64_t nv, int v_count,
+                       int32_t* flags, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

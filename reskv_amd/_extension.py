@@ -368,6 +368,18 @@ def kmeans_assign(x, centers, value=False):
     return ids
 
 
+def ids_in_range(pairs):
+    """[whether every id is in [0, count)] for two (int32 ids, count) pairs on one
+    GPU, from one launch and one synchronisation."""
+    (ki, kn), (vi, vn) = pairs
+    dev = _dev_check(ki, vi)
+    with torch.cuda.device(dev):
+        flags = torch.zeros(2, dtype=torch.int32, device=dev)
+        _lib.check(_lib.lib().reskv_ids_in_range(ki.data_ptr(), ki.numel(), int(kn), vi.data_ptr(), vi.numel(), int(vn),
+                                                 flags.data_ptr(), _stream(dev)), "ids_in_range")
+        return [not f for f in flags.tolist()]
+
+
 # ---------------------------------------------------------------------------
 # decode families
 # ---------------------------------------------------------------------------

@@ -62,6 +62,7 @@ SIGNATURES = {
                                  _i, _i, _f, _i, _vp, _vp, _vp, _i, _i, _vp, _vp, _i64, _vp]),
     "reskv_decode_recent_noalloc": (_i, [_vp, ctypes.POINTER(CTensor), ctypes.POINTER(CTensor), _vp, _vp, _i, _i,
                                          _i, _i, _i, _i, _f, _i, _vp, _vp, _vp, _i, _i, _vp, _vp]),
+    "reskv_ids_in_range": (_i, [_vp, _i64, _i, _vp, _i64, _i, _vp, _vp]),
     "reskv_ring_append": (_i, [_vp] * 7 + [_i] * 4 + [_vp]),
     "reskv_rope_table": (_i, [_vp, _i, _vp, _vp]),
     "reskv_merge_recent_scores": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp]),

@@ -14,7 +14,7 @@ the previous cache's tables, or fresh K-means), encode, append.
 
 import torch
 
-from ._extension import load_extension
+from ._extension import ids_in_range, load_extension
 from .config import KernelPlan, ResKVKernelConfig
 from .tensors import CompressedKV, CompressedTensor
 
@@ -157,7 +157,6 @@ def _external_rules(centers: torch.Tensor, ids: torch.Tensor, key: torch.Tensor,
            "external clustering has incompatible sizes")
     yield centers.device != key.device or ids.device != key.device, "external clustering must share the K/V device"
     yield ids.dtype not in _ID_DTYPES, "cluster IDs must be integer tensors"
-    yield bool(((ids < 0) | (ids >= centers.shape[2])).any()), "external cluster IDs are out of range"
 
 
 def _enforce(rules):
@@ -166,11 +165,34 @@ def _enforce(rules):
             raise ValueError(message)
 
 
+def _enforce_ranges(pairs):
+    """Every id of each (centres, ids) pair names a centre."""
+    native = len(pairs) == 2 and all(i.is_cuda and i.dtype == torch.int32 and i.is_contiguous() for _, i in pairs)
+    if native and pairs[0][1].device == pairs[1][1].device:
+        good = ids_in_range([(i, c.shape[2]) for c, i in pairs])
+    else:
+        good = (not bool(((i < 0) | (i >= c.shape[2])).any()) for c, i in pairs)
+    _enforce((not ok, "external cluster IDs are out of range") for ok in good)
+
+
+def _enforce_external(clustering, key, config):
+    """The rules of an external clustering, tensor by tensor (a tensor's ids are
+    checked before the next tensor's rules, all in one launch when they hold)."""
+    checked = []
+    for centers, ids in clustering:
+        try:
+            _enforce(_external_rules(centers, ids, key, config))
+        except ValueError:
+            _enforce_ranges(checked)
+            raise
+        checked.append((centers, ids))
+    _enforce_ranges(checked)
+
+
 def _clusters(key, value, config, previous, clustering):
     """((K centres, K ids), (V centres, V ids)) from the one source given."""
     if clustering is not None:
-        for centers, ids in clustering:
-            _enforce(_external_rules(centers, ids, key, config))
+        _enforce_external(clustering, key, config)
         return clustering
     if previous is not None:
         return (_incremental_cluster(key, previous.key.centroids, config),
