@@ -474,53 +474,52 @@ __device__ __forceinline__ void residual_f(const StageView<F>& S, const Prefetch
     }
 }
 
-// Signed INT4 / INT2 codes of the lane's channel pairs as exact fp16 pairs
-// (h[i] = values 2i, 2i + 1), without the scale.  Codes are biased to
-// unsigned fields by flipping their sign bits (u = code + 2^(bits-1)).  One
-// byte permute copies the pair's byte under an fp16 high byte 0x64 into both
-// halves (0x64bb: 1024 + bb, ulp 1); a mask keeps one field per half, which
-// then reads 1024 + u * 2^k for the field's bit offset k within the byte; one
-// packed fp16 FMA scales by 2^-k and subtracts 1024 / 2^k + 2^(bits-1),
-// leaving the code.  Every step is exact.
+// Signed INT4 / INT2 codes of the lane's channels as exact fp16 values, without the
+// scale; h[i] holds two channels of one word that lie half a word apart, because one
+// mask then takes both fields of the pair (code_channel says which).  Codes are
+// biased to unsigned fields by flipping their sign bits (u = code + 2^(bits-1)).
+// Two instructions a pair and two a word; pairs of neighbours, byte permutes under a
+// 0x64 high byte, a mask and a packed FMA, took three a pair and one a word.  29 of 330
+// VALU instructions a tile; B = 8, T = 16384, INT4: 65.3 -> 64.7 us (the VALU is busy
+// 69% of the time, the LDS 53%, the matrix cores 17%).
 template <int F>
 __device__ __forceinline__ void code_halves(const StageView<F>& S, const Prefetch<F>& R, int t, int g, uint32_t* h) {
-    constexpr uint32_t kMagic = 0x64646464u;
     uint32_t lw[4];
     lane_words<F>(S, t, g, lw);
-    if constexpr (F == D_Q4) {
-        // channel d in word d / 8 at bits 4 (d % 8): pair i of a word is its
-        // byte i, low nibble first (reference.py:17-21); words 2g, 2g + 1 hold
-        // channels 16g..16g+15 and words 8 + 2g, 9 + 2g channels 64+16g..64+16g+15
-        const half2_t mul = {(_Float16)1.0f, (_Float16)0.0625f}, add = {(_Float16)-1032.0f, (_Float16)-72.0f};
-        const uint32_t w[4] = {lw[0], lw[1], lw[2], lw[3]};
+    // field f of both 16-bit halves of x (BITS bits each) as fp16: under an exponent
+    // of 2^(10 - BITS f) the field's lowest bit counts as one, so that the or makes
+    // 2^(10 - BITS f) + u exactly, and one packed add takes the offsets off
+    constexpr int BITS = F == D_Q4 ? 4 : 2, N = 16 / BITS;  // pairs per word
+    constexpr int DIRECT = 1 + (10 - BITS) / BITS;          // fields within the 10 mantissa bits
+    static_assert(N <= 2 * DIRECT, "one shift reaches the rest");
+    constexpr uint32_t kField = (1u << BITS) - 1u;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t x = w[k] ^ 0x88888888u;
+    for (int k = 0; k < 16 / N; ++k) {
+        const uint32_t x = lw[k], y = x >> (BITS * DIRECT);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t d = __builtin_amdgcn_perm(kMagic, x, 0x04000400u + 0x00010001u * (uint32_t)j);
-                const half2_t e = __builtin_bit_cast(half2_t, d & 0xFFF0FF0Fu);  // 1024 + u0 | 1024 + 16 u1
-                h[4 * k + j] = __builtin_bit_cast(uint32_t, e * mul + add);
-            }
-        }
-    } else {
-        // channel d in word d / 16 at bits 2 (d % 16): pair p of a word is its
-        // nibble p; word g holds channels 16g..16g+15, word 4 + g 64+16g..
-        const half2_t mul_e = {(_Float16)1.0f, (_Float16)0.25f}, add_e = {(_Float16)-1026.0f, (_Float16)-258.0f};
-        const half2_t mul_o = {(_Float16)0.0625f, (_Float16)0.015625f}, add_o = {(_Float16)-66.0f, (_Float16)-18.0f};
-        const uint32_t w[2] = {lw[0], lw[1]};
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const uint32_t x = w[k] ^ 0xAAAAAAAAu;
-#pragma unroll
-            for (int p = 0; p < 8; ++p) {
-                const uint32_t d = __builtin_amdgcn_perm(kMagic, x, 0x04000400u + 0x00010001u * (uint32_t)(p >> 1));
-                // even nibble: fields at bits 0-1 and 2-3 of the byte; odd: 4-5 and 6-7
-                const half2_t e = __builtin_bit_cast(half2_t, d & ((p & 1) ? 0xFFC0FF30u : 0xFF0CFF03u));
-                h[8 * k + p] = __builtin_bit_cast(uint32_t, (p & 1) ? e * mul_o + add_o : e * mul_e + add_e);
-            }
+        for (int j = 0; j < N; ++j) {
+            const int f = j % DIRECT;
+            const uint32_t mask = 0x00010001u * (kField << (BITS * f));
+            const uint32_t base = 0x00010001u * (((25u - BITS * f) << 10) | (1u << (BITS * f + BITS - 1)));
+            const uint32_t d = __builtin_amdgcn_bitop3_b32(j < DIRECT ? x : y, mask, base, 0x6A);  // (a & b) ^ c
+            const _Float16 off = (_Float16)(-(float)(1 << (10 - BITS * f)) - (float)(1 << (BITS - 1)));
+            h[N * k + j] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, d) + (half2_t){off, off});
         }
     }
+}
+
+// The lane's channel of half `half` of h[i] from code_halves (0..31, in the order of
+// key_values), and the channel in column `col` of a V tile filled in that order.
+template <int F>
+constexpr int code_channel(int i, int half) {
+    constexpr int N = F == D_Q4 ? 4 : 8;
+    return i / N * (2 * N) + i % N + N * half;
+}
+template <int F>
+__device__ __forceinline__ int tile_channel(int col) {
+    if constexpr (F != D_Q4 && F != D_Q2) return col;
+    constexpr int N = F == D_Q4 ? 4 : 8;
+    return (col & ~(2 * N - 1)) | ((col & (2 * N - 1)) >> 1) | ((col & 1) * N);
 }
 
 // Key values of the lane's 32 channels (pre-RoPE, fp32): centroid + residual.
@@ -558,8 +557,9 @@ __device__ __forceinline__ void key_values(const StageView<F>& S, const Prefetch
         const float sc = h2f(R.sc);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            x[2 * i] = __builtin_fmaf(half_lo(h[i]), sc, half_lo(c[i]));
-            x[2 * i + 1] = __builtin_fmaf(half_hi(h[i]), sc, half_hi(c[i]));
+            const int lo = code_channel<F>(i, 0), hi = code_channel<F>(i, 1);
+            x[lo] = __builtin_fmaf(half_lo(h[i]), sc, lo & 1 ? half_hi(c[lo >> 1]) : half_lo(c[lo >> 1]));
+            x[hi] = __builtin_fmaf(half_hi(h[i]), sc, hi & 1 ? half_hi(c[hi >> 1]) : half_lo(c[hi >> 1]));
         }
     } else {
         float r[32];
@@ -1041,11 +1041,12 @@ decode_partial_kernel(DParams P) {
     for (int g = 0; g < G; ++g) bt[g] = VT::CENT ? 0.5f * accb[g >> 2][g & 3] : 0.0f;  // one-hot entries were 2
     __syncthreads();  // centroid table and stages no longer needed
     float* rec = reinterpret_cast<float*>(smem) + wave * G * kPartStride;
+    const int channel = tile_channel<VF>(lane);
 #pragma unroll
     for (int g = 0; g < G; ++g) {
         float* e = rec + g * kPartStride;
-        e[lane] = acc[g >> 2][0][g & 3];
-        e[64 + lane] = acc[g >> 2][1][g & 3];
+        e[channel] = acc[g >> 2][0][g & 3];
+        e[64 + channel] = acc[g >> 2][1][g & 3];
         e[kDim + lane] = bt[g];
         if (lane == 0) {
             e[kDim + kMaxClusters] = mt[g];
