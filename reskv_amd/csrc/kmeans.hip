@@ -272,8 +272,10 @@ __device__ __forceinline__ int sub_of(int j, int e) { return j + (e < 2 ? 4 : 0)
 // Bound: reading the rows and the VALU work (argmin, one-hot operands) take about
 // 0.1 ms each per iteration of 256 problems x 8128 tokens and overlap through four
 // independent four-wave workgroups per CU (128 VGPRs, 34 KB of LDS).  The whole
-// K-means of that size, 10 iterations: 2330 -> 1556 us; 16 problems x 8192: 214 ->
-// 184 us; 48 problems x 1999, C = 48, 15 iterations: 444 -> 329 us.  The kernel
+// K-means of that size, 10 iterations: 2330 -> 1556 us (1479 with the update below);
+// 16 problems x 8192: 214 -> 182 us; 48 problems x 1999, C = 48, 15 iterations:
+// 444 -> 329 us (288).  Two groups of waves per chunk (half the turns) measured
+// slower on 512 to 2048 workgroups: 189 against 182 us, 316 against 274.  The kernel
 // before had eight waves reduce 16 KB sums each through LDS for every chunk, wrote
 // a 16 KB partial per 64 KB of tokens, and (C > 32) fitted one workgroup per CU.
 template <int NB, bool LO, int G>

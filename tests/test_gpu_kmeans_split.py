@@ -29,3 +29,27 @@ def test_results_do_not_depend_on_the_split(device, t, count):
     (kc, ki), (vc, vi) = kmeans_kv(base, base.flip(1).contiguous(), None, None, 4, count)
     k1, v1 = kmeans(base, None, 4, False, count), kmeans(base.flip(1).contiguous(), None, 4, True, count)
     assert torch.equal(kc, k1[0]) and torch.equal(ki, k1[1]) and torch.equal(vc, v1[0]) and torch.equal(vi, v1[1])
+
+
+@pytest.mark.parametrize("problems,t,count", [(40, 2339, 8), (40, 2339, 16), (24, 3000, 17), (144, 1100, 16)])
+def test_many_problems_follow_lloyd(device, problems, t, count):
+    """K against a 64-bit Lloyd loop on grids of more than one workgroup per CU, at
+    the smallest centre tables (an earlier kernel read its tables past its LDS there,
+    and gave wrong ids without any error).  Gaussian tokens on 128 channels: two fp32
+    distances are closer than their rounding for fewer than one token in 1000."""
+    from reskv_amd._extension import kmeans
+
+    g = seeded(count + t)
+    x = (torch.randn(problems, t, 128, generator=g) * torch.exp(torch.randn(problems, 1, 128, generator=g))).half()
+    x = x.to(device)
+    centres, ids = kmeans(x, None, 3, False, count)
+    wide = x.double()
+    c = wide[:, torch.linspace(0, t - 1, count).long()]
+    for _ in range(3):
+        near = ((c * c).sum(-1)[:, None] - 2 * torch.bmm(wide, c.transpose(1, 2).contiguous())).argmin(-1)
+        member = torch.nn.functional.one_hot(near, count).double().transpose(1, 2).contiguous()
+        n = member.sum(-1, keepdim=True)
+        c = torch.where(n > 0, torch.bmm(member, wide) / n.clamp(min=1), c)
+    assert (near != ids).float().mean().item() < 1e-3
+    # centres are returned in fp16: half a unit in the last place below 4 is 1e-3
+    assert (centres.double() - c).abs().median().item() < 2e-3
