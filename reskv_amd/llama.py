@@ -101,6 +101,13 @@ def _on_gpu(*tensors):
     _need(all(t is None or t.is_cuda for t in tensors), "every tensor must be a CUDA tensor")
 
 
+def _launch(name, ref, *args):
+    """Calls the library's ``name`` on the current stream of ref's GPU, made the current one
+    meanwhile: a launch goes to the current device, whatever the device of its pointers."""
+    with torch.cuda.device(ref.device):
+        _lib.check(getattr(_lib.lib(), name)(*args, _stream(ref)), name)
+
+
 def fused_rmsnorm(x, w, eps, out):
     """``_rmsnorm`` of fp16 rows x [R, hidden] into out, one launch."""
     _fp16_rows("x", x)
@@ -108,8 +115,7 @@ def fused_rmsnorm(x, w, eps, out):
     _need(w.dtype == torch.float16 and w.is_contiguous() and w.numel() == x.shape[1],
           "w must be a contiguous fp16 vector of the hidden size")
     _on_gpu(x, w, out)
-    _lib.check(_lib.lib().reskv_llama_rmsnorm(x.data_ptr(), w.data_ptr(), out.data_ptr(), x.shape[0], x.shape[1],
-                                              eps, _stream(x)), "reskv_llama_rmsnorm")
+    _launch("reskv_llama_rmsnorm", x, x.data_ptr(), w.data_ptr(), out.data_ptr(), x.shape[0], x.shape[1], eps)
     return out
 
 
@@ -118,8 +124,7 @@ def fused_silu_mul(gu, out):
     _fp16_rows("out", out)
     _fp16_rows("gu", gu, out.shape[0], 2 * out.shape[1])
     _on_gpu(gu, out)
-    _lib.check(_lib.lib().reskv_llama_silu_mul(gu.data_ptr(), out.data_ptr(), gu.shape[0], out.shape[1],
-                                               _stream(gu)), "reskv_llama_silu_mul")
+    _launch("reskv_llama_silu_mul", gu, gu.data_ptr(), out.data_ptr(), gu.shape[0], out.shape[1])
     return out
 
 
@@ -151,10 +156,9 @@ def fused_qkv_rope(qkv, cos, sin, pos, q, qr, k, kr, v, targets=None):
 
     _on_gpu(qkv, cos, sin, pos, q, qr, k, kr, v, rot, raw, vc, slot)
     ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-    _lib.check(_lib.lib().reskv_llama_qkv_rope(
-        qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), b, hq, hk, q.data_ptr(), qr.data_ptr(),
-        k.data_ptr(), kr.data_ptr(), v.data_ptr(), ptr(rot), ptr(raw), ptr(vc), ptr(slot), *strides,
-        _stream(qkv)), "reskv_llama_qkv_rope")
+    _launch("reskv_llama_qkv_rope", qkv, qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), b, hq, hk,
+            q.data_ptr(), qr.data_ptr(), k.data_ptr(), kr.data_ptr(), v.data_ptr(), ptr(rot), ptr(raw), ptr(vc),
+            ptr(slot), *strides)
 
 
 def fused_prefill_split(qkv, cos, sin, batch, heads, kv_heads):
@@ -168,9 +172,8 @@ def fused_prefill_split(qkv, cos, sin, batch, heads, kv_heads):
     _on_gpu(qkv, cos, sin)
     new = lambda h: torch.empty(batch, h, t, 128, dtype=torch.float16, device=qkv.device)  # noqa: E731
     qr, k, kr, v = new(heads), new(kv_heads), new(kv_heads), new(kv_heads)
-    _lib.check(_lib.lib().reskv_llama_prefill_split(
-        qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), batch, t, heads, kv_heads, qr.data_ptr(), k.data_ptr(),
-        kr.data_ptr(), v.data_ptr(), _stream(qkv)), "reskv_llama_prefill_split")
+    _launch("reskv_llama_prefill_split", qkv, qkv.data_ptr(), cos.data_ptr(), sin.data_ptr(), batch, t, heads,
+            kv_heads, qr.data_ptr(), k.data_ptr(), kr.data_ptr(), v.data_ptr())
     return qr, k, kr, v
 
 
@@ -184,9 +187,8 @@ def fused_prefill_attention(q, k, v, scaling):
     _need(_prefill_ratio(hq, k.shape[1]), "the query/KV head ratio must be 1, 2 or a multiple of 4")
     _on_gpu(q, k, v)
     out = torch.empty(b, t, hq, 128, dtype=torch.float16, device=q.device)
-    _lib.check(_lib.lib().reskv_llama_prefill_attention(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, hq, k.shape[1], t, float(scaling), _stream(q)),
-        "reskv_llama_prefill_attention")
+    _launch("reskv_llama_prefill_attention", q, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, hq,
+            k.shape[1], t, float(scaling))
     return out
 
 
