@@ -520,6 +520,9 @@ class StepDecoder:
         elements) when given, else a buffer reused by the next call.  With a
         recent window the split merge joins it in the same launch
         (``reskv_decode_recent``)."""
+        if torch._C._cuda_getDevice() != self.dev.index:  # a launch goes to the current device
+            with torch.cuda.device(self.dev):
+                return self.run(query, position, query_rot, ring_k, ring_v, ring_len, ring_stride, out)
         L = _lib.lib()
         stream = _stream(self.dev)
         if out is not None:

@@ -419,6 +419,10 @@ class GreedyDecoder:
         """Records the fixed-shape parts once (after a warm-up on a side stream).
         The warm-up appends layer 0's token at this step's slot, which the
         step's own append then overwrites with the same values."""
+        with torch.cuda.device(self.x.device):
+            self._capture()
+
+    def _capture(self):
         self._set_slots()
         x0, tok0 = self.x.clone(), self.tok.clone()
         side = torch.cuda.Stream(device=self.model.device)
@@ -465,6 +469,10 @@ class GreedyDecoder:
         ``events`` (list) collects (before, after) CUDA events around each attention."""
         if self.pos >= self.max_pos:
             raise RuntimeError("decoder capacity exhausted")
+        with torch.cuda.device(self.x.device):  # graphs, streams and events are the current device's
+            return self._step(events)
+
+    def _step(self, events):
         if self.graphs is None:
             self.capture()
         self._set_slots()

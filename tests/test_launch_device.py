@@ -57,3 +57,35 @@ def test_fused_steps_make_their_tensors_device_current(library):
     cpu = torch.device("cpu")
     assert library.calls == [("reskv_llama_" + n, cpu) for n in
                              ("rmsnorm", "silu_mul", "qkv_rope", "prefill_split", "prefill_attention")]
+
+
+def test_step_decoder_makes_its_device_current(library, monkeypatch):
+    from reskv_amd import _extension
+
+    monkeypatch.setattr(_extension._lib, "lib", lambda: library)
+    monkeypatch.setattr(_extension, "_stream", lambda d: 0)
+    # device 1 current until the decoder switches to its own (the CPU's index is None)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: None if library.entered else 1, raising=False)
+    cpu = torch.device("cpu")
+    step = object.__new__(_extension.StepDecoder)
+    step.dev, step.b, step.nh, step.kh, step.t, step.scaling, step.splits = cpu, 1, 4, 1, 16, 0.1, 0
+    step.kdesc = step.vdesc = None
+    step.freq = step.table = step.m = step.l = torch.zeros(4)
+    step.ws = torch.zeros(4, dtype=torch.uint8)
+    step.out, step.merged = torch.zeros(4, 128, **f16), torch.zeros(4, 128, **f16)
+    q = torch.zeros(1, 4, 1, 128, **f16)
+    ring = torch.zeros(1, 1, 8, 128, **f16)
+    assert step.run(q, 20).shape == (1, 4, 1, 128)
+    assert step.run(q, 20, q, ring, ring, 3, 8).shape == (1, 4, 1, 128)
+    assert library.calls == [("reskv_decode_rope", cpu), ("reskv_decode_recent", cpu)]
+
+
+def test_greedy_decoder_steps_and_captures_on_its_device(library):
+    seen = []
+    dec = object.__new__(llama.GreedyDecoder)
+    dec.x, dec.pos, dec.max_pos = torch.zeros(1, 8), 0, 2
+    dec._step = lambda events: seen.append(("step", library.entered[-1]))
+    dec._capture = lambda: seen.append(("capture", library.entered[-1]))
+    dec.step()
+    dec.capture()
+    assert seen == [("step", torch.device("cpu")), ("capture", torch.device("cpu"))]
