@@ -587,19 +587,23 @@ _RING_STRIDES = ctypes.c_int64 * 6
 
 def ring_append(rings, tokens, slot):
     """Writes one token's rows (three [B, H, 1, 128] tensors) to token ``slot`` of the
-    three contiguous ring buffers [B, H, cap, 128], one launch.  Returns False, having
-    done nothing, for tensors that torch's copies have to take: other shapes, types,
-    devices or alignments, gradients, or a call that is being compiled."""
+    three ring buffers [B, H, cap, 128], one launch.  Returns False, having done nothing,
+    for tensors that torch's copies have to take: tokens or rings of other shapes, types,
+    devices, layouts or alignments, gradients, or a call that is being compiled."""
     ring = rings[0]
     if not ring.is_cuda or ring.element_size() != 2 or ring.shape[3] != 128 or torch.compiler.is_compiling():
         return False
     dev = ring.device
     if torch._C._cuda_getDevice() != dev.index:
         return False
-    b, h, cap, _ = ring.shape
-    strides = []
+    shape, dtype = ring.shape, ring.dtype
+    b, h, cap, _ = shape
+    for r in rings:  # the kernel indexes all three as dense buffers of one shape
+        if r.shape != shape or r.dtype != dtype or r.device != dev or not r.is_contiguous() or r.data_ptr() % 16:
+            return False
+    strides, row = [], (b, h, 1, 128)
     for x in tokens:
-        if x.shape != (b, h, 1, 128) or x.dtype != ring.dtype or x.device != dev or x.requires_grad:
+        if x.shape != row or x.dtype != dtype or x.device != dev or x.requires_grad:
             return False
         sb, sh, _, sd = x.stride()
         if sd != 1 or sb % 8 or sh % 8 or x.data_ptr() % 16:
