@@ -21,6 +21,9 @@ from functools import lru_cache
 from types import SimpleNamespace
 
 import torch
+import torch.autograd.forward_ad as _forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from .config import KernelPlan
@@ -43,6 +46,20 @@ def _ptr(t):
 
 def _stream(device):
     return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+def eager():
+    """Whether torch runs each operation as it is called, with nothing beside the kernels
+    that has to see it: no compilation, tracing, functional transform, forward-mode
+    level, and no dispatch or function mode (the default device's concerns new tensors
+    only).  A native launch in the place of torch operations on a caller's tensors is one
+    that these would miss."""
+    c = torch._C
+    if c._len_torch_function_stack() and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()):
+        return False
+    return not (c._len_torch_dispatch_stack() or _forward_ad._current_level >= 0
+                or c._functorch.maybe_current_level() is not None or c._get_tracing_state() is not None
+                or torch.compiler.is_compiling())
 
 
 def _dev_check(*tensors, contiguous=True):
@@ -589,29 +606,38 @@ def ring_append(rings, tokens, slot):
     """Writes one token's rows (three [B, H, 1, 128] tensors) to token ``slot`` of the
     three ring buffers [B, H, cap, 128], one launch.  Returns False, having done nothing,
     for tensors that torch's copies have to take: tokens or rings of other shapes, types,
-    devices, layouts or alignments, gradients, or a call that is being compiled."""
+    devices, layouts or alignments, subclasses, gradients, inference tensors outside
+    inference mode (which the copies refuse), or a call that something has to see."""
     ring = rings[0]
-    if not ring.is_cuda or ring.element_size() != 2 or ring.shape[3] != 128 or torch.compiler.is_compiling():
-        return False
-    dev = ring.device
-    if torch._C._cuda_getDevice() != dev.index:
+    index = ring.get_device()
+    if not ring.is_cuda or ring.element_size() != 2 or torch._C._cuda_getDevice() != index or not eager():
         return False
     shape, dtype = ring.shape, ring.dtype
-    b, h, cap, _ = shape
-    for r in rings:  # the kernel indexes all three as dense buffers of one shape
-        if r.shape != shape or r.dtype != dtype or r.device != dev or not r.is_contiguous() or r.data_ptr() % 16:
-            return False
-    strides, row = [], (b, h, 1, 128)
+    b, h, cap, width = shape
+    if width != 128:
+        return False
+    followed, inference = torch.is_grad_enabled(), torch.is_inference_mode_enabled()
+    pointers, strides, row = [], [], (b, h, 1, 128)
     for x in tokens:
-        if x.shape != row or x.dtype != dtype or x.device != dev or x.requires_grad:
+        if x.shape != row or x.dtype != dtype or x.get_device() != index or type(x) is not torch.Tensor or x.is_neg():
             return False
         sb, sh, _, sd = x.stride()
-        if sd != 1 or sb % 8 or sh % 8 or x.data_ptr() % 16:
+        at = x.data_ptr()
+        if sd != 1 or sb % 8 or sh % 8 or at % 16 or (followed and x.requires_grad):
             return False
         strides += (sb, sh)
-    _lib.check(_lib.lib().reskv_ring_append(
-        tokens[0].data_ptr(), tokens[1].data_ptr(), tokens[2].data_ptr(), _RING_STRIDES(*strides),
-        rings[0].data_ptr(), rings[1].data_ptr(), rings[2].data_ptr(), b, h, cap, slot, _stream(dev)), "ring_append")
+        pointers.append(at)
+    for r in rings:  # the kernel indexes all three as dense buffers of one shape
+        at = r.data_ptr()
+        if (r.shape != shape or r.dtype != dtype or r.get_device() != index or type(r) is not torch.Tensor
+                or not r.is_contiguous() or at % 16 or (followed and r.requires_grad)
+                or (r.is_inference() and not inference)):
+            return False
+        pointers.append(at)
+    k, raw, v, rk, rraw, rv = pointers
+    _lib.check(_lib.lib().reskv_ring_append(k, raw, v, _RING_STRIDES(*strides), rk, rraw, rv, b, h, cap, slot,
+                                            _stream(ring.device)), "ring_append")
+    torch.autograd.graph.increment_version(rings)  # as an in-place copy does
     return True
 
 

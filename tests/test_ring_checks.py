@@ -4,6 +4,10 @@ Everything else has to be left to torch's copies, which handle (or refuse) it.""
 
 import pytest
 import torch
+import torch.autograd.forward_ad as forward_ad
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from reskv_amd import _extension
 
@@ -22,7 +26,7 @@ def append(monkeypatch):
             return 0
 
     monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
-    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: None, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: -1, raising=False)
     monkeypatch.setattr(_extension, "_stream", lambda d: 0)
     monkeypatch.setattr(_extension._lib, "lib", lambda: Library())
 
@@ -62,3 +66,69 @@ def test_every_ring_is_one_dense_buffer_of_the_same_kind(append, which, form):
         "misaligned": lambda: torch.zeros(x.numel() + 1, **f16)[1:].view(x.shape),
     }[form]()
     assert not append(rings, _tokens())
+
+
+class _Subclass(torch.Tensor):
+    pass
+
+
+class _Dispatch(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+class _Function(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("form", ["fake", "subclass", "negated", "gradient"])
+def test_tokens_that_are_not_plain_values_are_left_to_torch(append, form):
+    for at in range(3):
+        tokens, rings = _tokens(), _rings()
+        if form == "fake":
+            with FakeTensorMode():
+                tokens[at] = torch.ones(2, 3, 1, 128, **f16)
+        elif form == "subclass":
+            tokens[at] = tokens[at].as_subclass(_Subclass)
+        elif form == "negated":
+            tokens[at] = torch._neg_view(tokens[at])
+        else:
+            tokens[at].requires_grad_()
+        assert not append(rings, tokens)
+
+
+def test_calls_that_something_has_to_see_are_left_to_torch(append):
+    rings, tokens = _rings(), _tokens()
+    for mode in (_Dispatch(), _Function(), FakeTensorMode(), forward_ad.dual_level()):
+        with mode:
+            assert not append(rings, tokens)
+    with torch.device("cpu"):  # a default device for new tensors
+        assert append(rings, tokens)
+
+    taken = []
+
+    def inside(x):
+        taken.append(append(rings, tokens))
+        return x * 2
+
+    torch.jit.trace(inside, torch.zeros(2), check_trace=False)
+    torch.func.vmap(inside)(torch.zeros(2, 2))
+    torch.func.functionalize(inside)(torch.zeros(2))
+    torch.func.jvp(inside, (torch.zeros(2),), (torch.ones(2),))
+    assert len(taken) >= 4 and not any(taken)
+    assert append(rings, tokens)
+
+
+def test_rings_that_autograd_follows_are_left_to_torch(append):
+    rings = _rings()
+    rings[1].requires_grad_()
+    assert not append(rings, _tokens())
+    with torch.inference_mode():
+        inner = _rings()
+        assert append(inner, _tokens())
+    assert not append(inner, _tokens())  # copies refuse an in-place update outside inference mode
+    plain = _rings()
+    before = [r._version for r in plain]
+    assert append(plain, _tokens())
+    assert all(r._version > v for r, v in zip(plain, before))
