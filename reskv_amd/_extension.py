@@ -606,15 +606,16 @@ def ring_append(rings, tokens, slot):
     """Writes one token's rows (three [B, H, 1, 128] tensors) to token ``slot`` of the
     three ring buffers [B, H, cap, 128], one launch.  Returns False, having done nothing,
     for tensors that torch's copies have to take: tokens or rings of other shapes, types,
-    devices, layouts or alignments, subclasses, gradients, inference tensors outside
-    inference mode (which the copies refuse), or a call that something has to see."""
+    devices, layouts or alignments, empty ones, tokens in a ring, subclasses, gradients,
+    inference tensors outside inference mode (which the copies refuse), or a call that
+    something has to see."""
     ring = rings[0]
     index = ring.get_device()
     if not ring.is_cuda or ring.element_size() != 2 or torch._C._cuda_getDevice() != index or not eager():
         return False
     shape, dtype = ring.shape, ring.dtype
     b, h, cap, width = shape
-    if width != 128:
+    if width != 128 or not 0 < b * h < 1 << 24 or not 0 <= slot < cap:  # the kernel's own bounds
         return False
     followed, inference = torch.is_grad_enabled(), torch.is_inference_mode_enabled()
     pointers, strides, row = [], [], (b, h, 1, 128)
@@ -635,6 +636,10 @@ def ring_append(rings, tokens, slot):
             return False
         pointers.append(at)
     k, raw, v, rk, rraw, rv = pointers
+    span = b * h * cap * 256
+    for at in (rk, rraw, rv):  # a token that lies in a ring: the copies write one after the other
+        if at <= k < at + span or at <= raw < at + span or at <= v < at + span:
+            return False
     _lib.check(_lib.lib().reskv_ring_append(k, raw, v, _RING_STRIDES(*strides), rk, rraw, rv, b, h, cap, slot,
                                             _stream(ring.device)), "ring_append")
     torch.autograd.graph.increment_version(rings)  # as an in-place copy does

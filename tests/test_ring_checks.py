@@ -132,3 +132,27 @@ def test_rings_that_autograd_follows_are_left_to_torch(append):
     before = [r._version for r in plain]
     assert append(plain, _tokens())
     assert all(r._version > v for r, v in zip(plain, before))
+
+
+@pytest.mark.parametrize("b,h", [(0, 3), (2, 0)])
+def test_an_empty_batch_is_left_to_torch(append, b, h):
+    assert not append(_rings(b, h), _tokens(b, h))
+
+
+def test_more_rows_than_the_kernel_indexes_are_left_to_torch(append):
+    rows = 1 << 24
+    ring = torch.empty(rows, 1, 1, 128, **f16)  # 4 GiB of addresses, no page of it touched
+    token = torch.empty(1, 1, 1, 128, **f16).expand(rows, 1, 1, 128)
+    assert not append([ring] * 3, [token] * 3)
+
+
+@pytest.mark.parametrize("slot", [-1, 8])
+def test_a_slot_past_the_ring_is_left_to_torch(append, slot):
+    assert not append(_rings(), _tokens(), slot)
+
+
+def test_tokens_that_lie_in_a_ring_are_left_to_torch(append):
+    # the copies run one after the other, the launch writes all three at once
+    rings, tokens = _rings(), _tokens()
+    tokens[1] = rings[0][:, :, 3:4]
+    assert not append(rings, tokens, 3)
