@@ -455,11 +455,12 @@ def _decode(Q, kdesc, vdesc, keep, nh_kv, nh, start_pos, pos_q, rope_base, scali
 def _described(t):
     """What a CompressedTensor's native views are to the library, without their
     addresses: (format, bits, centroids, width, token row stride, centroid row
-    stride, has metadata, has scale).  The views are checked when they are made and
-    are not replaced afterwards, so this is worked out once for each set of them."""
+    stride, has metadata, has scale).  It follows from the views, which are made and
+    checked with the tensor, and from the plan, and is worked out again when either
+    has been replaced."""
     known = t.__dict__.get("_layout")
-    if known is not None and known[0] is t._native:
-        return known[1]
+    if known is not None and known[0] is t._native and known[1] is t.plan:
+        return known[2]
     c, i, p, m, sc = t._native
     plan = t.plan
     if plan.bits == 16 and plan.layout == "unstructured":
@@ -471,8 +472,9 @@ def _described(t):
     else:
         fmt, bits, m = _lib.FMT_QUANT, int(plan.bits), None
     d = _ctensor(c, i, p, m, sc, fmt, bits)
-    t._layout = (t._native, (d.format, d.bits, d.nc, d.width, d.t_stride, d.c_stride, m is not None, sc is not None))
-    return t._layout[1]
+    t._layout = (t._native, plan, (d.format, d.bits, d.nc, d.width, d.t_stride, d.c_stride, m is not None,
+                                   sc is not None))
+    return t._layout[2]
 
 
 def _descriptor(t):
