@@ -573,11 +573,13 @@ def decode_step(query2d, cache, num_q_heads, *, position, start_position, scalin
     output (``reskv_decode_recent``), so a step is two kernel launches.
     """
     dev = query2d.device
-    _require(query2d.is_cuda and cache.key.payload.device == dev and cache.value.payload.device == dev,
-             "all tensors must be on the same GPU")
+    index = query2d.get_device()
+    for x in cache.key._native + cache.value._native:
+        _require(x is None or x.get_device() == index, "all tensors must be on the same GPU")
+    _require(query2d.is_cuda, "all tensors must be on the same GPU")
     if recent is not None:
         _dev_check(query2d, *recent)
-    if torch._C._cuda_getDevice() != dev.index:
+    if torch._C._cuda_getDevice() != index:
         with torch.cuda.device(dev):
             return decode_step(query2d, cache, num_q_heads, position=position, start_position=start_position,
                                scaling=scaling, inv_freq=inv_freq, rope_theta=rope_theta, splits=splits,
