@@ -588,7 +588,7 @@ def decode_step(query2d, cache, num_q_heads, *, position, start_position, scalin
     nh, t, splits = int(num_q_heads), cache.seq_len, int(splits)
     freq, table = _rope(inv_freq, rope_theta, dev, int(start_position) + t)
     L = _lib.lib()
-    out = torch.empty_like(query2d)
+    out = _empty((b * nh, 128), torch.float16, dev)  # plain, also for a subclass's query
     ws = _workspace(L.reskv_decode_workspace_bytes(b, nh, kh, t, splits), dev)
     common = (query2d.data_ptr(), _descriptor(cache.key), _descriptor(cache.value), freq.data_ptr(),
               table.data_ptr(), b, nh, kh, t, int(start_position), int(position), float(scaling), splits)

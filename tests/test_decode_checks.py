@@ -75,3 +75,12 @@ def test_every_view_is_on_the_querys_device(decode, side, which):
     with pytest.raises(RuntimeError, match="same GPU"):
         call(query, cache)
     assert len(calls) == 1
+
+
+def test_the_result_is_a_plain_tensor_whatever_the_query_is(decode):
+    class Subclass(torch.Tensor):
+        pass
+
+    query = torch.zeros(4, 128, dtype=torch.float16).as_subclass(Subclass)
+    out = decode[0](query, CompressedKV(_tensor(), _tensor()))
+    assert type(out) is torch.Tensor and out.dtype == torch.float16 and out.is_contiguous()
