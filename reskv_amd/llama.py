@@ -32,7 +32,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib
-from ._extension import dense_decode
+from ._extension import dense_decode, eager
 from .cache import ResKVLayerCache
 from .config import ResKVKernelConfig
 
@@ -255,10 +255,12 @@ class RandomLlama:
             flat[r0: r0 + rows] += F.linear(act, p["wd"])
 
     def _fused(self, t):
-        """Whether the library's kernels take this model's prompts (else torch formulas)."""
+        """Whether the library's kernels take this model's prompts (else torch formulas,
+        also where something has to see the operations)."""
         s = self.shape
         return (self.device.type == "cuda" and s.head_dim == 128 and _prefill_ratio(s.heads, s.kv_heads)
-                and s.hidden % 8 == 0 and s.hidden <= 8192 and s.ffn % 8 == 0 and t <= 1 << 22)
+                and s.hidden % 8 == 0 and s.hidden <= 8192 and s.ffn % 8 == 0 and t <= 1 << 22
+                and eager())
 
     def _layer_fused(self, li, p, x, cos, sin, sink, rows=16384):
         """One layer of the prompt in place on x [B, T, hidden]: the norms, the split and

@@ -4,8 +4,11 @@ library (shape, dtype and layout first, then the device)."""
 
 import pytest
 import torch
+import torch.autograd.forward_ad as forward_ad
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
 
-from reskv_amd.llama import fused_qkv_rope, fused_rmsnorm, fused_silu_mul
+from reskv_amd.llama import LlamaShape, RandomLlama, fused_qkv_rope, fused_rmsnorm, fused_silu_mul
 
 f16 = dict(dtype=torch.float16)
 
@@ -76,3 +79,28 @@ def test_qkv_rope_append_target_checks():
         fused_qkv_rope(**args, targets=(torch.zeros(2, 2, 16, 128, **f16), None, None, slot))
     with pytest.raises(ValueError, match="CUDA"):
         fused_qkv_rope(**args, targets=(cache, cache, cache, slot))
+
+
+def _cuda_model():
+    model = object.__new__(RandomLlama)
+    model.shape, model.device, model.scaling = LlamaShape(), torch.device("cuda", 0), 128 ** -0.5
+    return model
+
+
+def test_prompts_that_torch_has_to_see_take_the_torch_formulas():
+    """Raw-pointer launches are not seen by tracing, modes, transforms or forward-mode levels."""
+    model = _cuda_model()
+    assert model._fused(64)
+    for mode in (FakeTensorMode(), forward_ad.dual_level()):
+        with mode:
+            assert not model._fused(64)
+    seen = []
+
+    def inside(x):
+        seen.append(model._fused(64))
+        return x * 2
+
+    torch.jit.trace(inside, torch.zeros(2), check_trace=False)
+    make_fx(inside)(torch.zeros(2))
+    torch.func.vmap(inside)(torch.zeros(2, 2))
+    assert len(seen) >= 3 and not any(seen)
