@@ -255,12 +255,15 @@ class RandomLlama:
             flat[r0: r0 + rows] += F.linear(act, p["wd"])
 
     def _fused(self, t):
-        """Whether the library's kernels take this model's prompts (else torch formulas,
-        also where something has to see the operations)."""
+        """Whether the library's kernels take this model's prompts (else torch formulas:
+        shapes, scalings and norm gains that the kernels refuse, and operations that
+        something has to see)."""
         s = self.shape
         return (self.device.type == "cuda" and s.head_dim == 128 and _prefill_ratio(s.heads, s.kv_heads)
                 and s.hidden % 8 == 0 and s.hidden <= 8192 and s.ffn % 8 == 0 and t <= 1 << 22
-                and eager())
+                and self.scaling > 0.0 and eager()
+                and all(w.dtype == torch.float16 and w.is_contiguous() and w.data_ptr() % 16 == 0
+                        for p in self.layers for w in (p["n1"], p["n2"])))
 
     def _layer_fused(self, li, p, x, cos, sin, sink, rows=16384):
         """One layer of the prompt in place on x [B, T, hidden]: the norms, the split and

@@ -84,6 +84,7 @@ def test_qkv_rope_append_target_checks():
 def _cuda_model():
     model = object.__new__(RandomLlama)
     model.shape, model.device, model.scaling = LlamaShape(), torch.device("cuda", 0), 128 ** -0.5
+    model.layers = []
     return model
 
 
@@ -104,3 +105,20 @@ def test_prompts_that_torch_has_to_see_take_the_torch_formulas():
     make_fx(inside)(torch.zeros(2))
     torch.func.vmap(inside)(torch.zeros(2, 2))
     assert len(seen) >= 3 and not any(seen)
+
+
+@pytest.mark.parametrize("scaling", [0.0, -0.5, float("nan")])
+def test_scalings_that_the_prompt_kernel_refuses_take_the_torch_formulas(scaling):
+    model = _cuda_model()
+    model.scaling = scaling
+    assert not model._fused(64)
+
+
+@pytest.mark.parametrize("name", ["n1", "n2"])
+@pytest.mark.parametrize("gains", [torch.ones(4096), torch.ones(8192, **f16)[::2], torch.ones(4104, **f16)[1:4097]])
+def test_norm_gains_that_the_kernel_refuses_take_the_torch_formulas(name, gains):
+    model = _cuda_model()
+    model.layers = [{n: torch.ones(4096, **f16) for n in ("n1", "n2")} for _ in range(2)]
+    assert model._fused(64)
+    model.layers[1][name] = gains
+    assert not model._fused(64)
