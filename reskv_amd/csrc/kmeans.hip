@@ -425,13 +425,15 @@ kmeans_assign_kernel(
             token_argmin(bd, bi);
         } else {
             if (vgroup) {
-                // decode groups: fp32(fp16(|x|^2 + |c|^2) - 2 <x, c>), lowest index on ties
-                float bd = INFINITY;
-                bi = 1 << 20;
+                // decode groups: fp32(fp16(|x|^2 + |c|^2) - 2 <x, c>), lowest index on
+                // ties, which all centres are for a token whose fp16 norm is infinite
+                float bd = fmaf(-2.0f, acc[0][0], h2f(f2h(xn + cn[0].x)));
+                bi = 0;
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
+                        if (nb == 0 && r == 0) continue;
                         const float e = h2f(f2h(xn + cnorm(cn[nb], r)));
                         const float d = fmaf(-2.0f, acc[nb][r], e);
                         const bool take = d < bd;
