@@ -115,7 +115,10 @@ __global__ void __launch_bounds__(kThreads, 2) prefill_attention_kernel(AttnArgs
     for (int db = 0; db < 4; ++db)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[db][i] = 0.0f;
-    float m = -INFINITY, l = 0.0f;  // log2-domain maximum; this lane's half of the weights' sum
+    // log2-domain maximum, and this lane's half of the weights' sum.  The maximum starts at
+    // the lowest finite value: scores of minus infinity then weigh exp2(-inf) = 0, where
+    // against a maximum of minus infinity they would give NaN
+    float m = -__FLT_MAX__, l = 0.0f;
     // transpose reads: lane i of a 16-lane row points at key i / 4, channel 4 (i % 4) of
     // its 4 x 16 block and receives the block's four keys of channel i
     const int i16 = lane & 15;
@@ -152,7 +155,6 @@ __global__ void __launch_bounds__(kThreads, 2) prefill_attention_kernel(AttnArgs
                 for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[kb2][i]);
             const auto sw = __builtin_amdgcn_permlane32_swap((uint32_t)f2i(mx), (uint32_t)f2i(mx), false, false);
             mx = fmaxf(i2f((int)sw[0]), i2f((int)sw[1])) * A.c;  // c > 0
-            // every query has a key in its first tile (key 0), so m is finite from then on
             if (ballot(mx > m) != 0) {
                 const float mn = fmaxf(m, mx);
                 const float alpha = __builtin_amdgcn_exp2f(m - mn);
