@@ -246,10 +246,13 @@ int reskv_decode_recent(const void* q, const reskv_ctensor* k, const reskv_ctens
  * that forbid hipMalloc).  The split-K partial records go to a file-scope
  * device array of RESKV_NOALLOC_SCRATCH_BYTES (8 MiB) that each GPU holds
  * until the process ends; its address is looked up once per device
- * (hipGetSymbolAddress) on the first call.  Sizes whose partials exceed it
- * (reskv_decode_workspace_bytes(B, Hq, H, T, splits) > 8 MiB; the automatic
- * split count stays below that up to B*Hq = 10,000 rows) are rejected with an
- * error.  The array used is the current device's: `stream` must belong to
+ * (hipGetSymbolAddress) on the first call.  Sizes whose partials can exceed it are
+ * rejected with an error: B * Hq records of 776 bytes per split, for
+ * min(splits, T, 1024) splits, or with an automatic count (splits <= 0) for
+ * min(ceil(1024 / (B * H)), T / 128) of them, at least one.  With an automatic
+ * count B * Hq + 1024 * Hq / H <= 10,810 is always accepted.  A call makes the
+ * splits that reskv_decode_recent makes.
+ * The array used is the current device's: `stream` must belong to
  * the current device (the null stream does), otherwise the call is rejected.
  * Every call on a GPU shares that GPU's array: calls that overlap on one GPU
  * race.  Arguments and result are those of reskv_decode_recent (Tr = 0:

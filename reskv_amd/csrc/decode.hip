@@ -1876,15 +1876,13 @@ extern "C" int reskv_decode_recent_noalloc(const void* q, const reskv_ctensor* k
                                            const void* q_rope, const void* k_recent, const void* v_recent, int Tr,
                                            int r_stride, void* out, void* stream) {
     RESKV_REQUIRE(B > 0 && Hq > 0 && H > 0 && T > 0, "batch, head and token counts must be positive");
-    int64_t need = reskv_decode_workspace_bytes(B, Hq, H, T, splits);
-    if (splits <= 0 && need > kNoAllocScratchBytes && T > kWaves * 2 * kTile) {
-        // one split less (whole pairs of tiles per wave) may still fit
-        const int whole = std::min(most_splits(B, H, T, kMaxGroupsPerCU), T / (kWaves * 2 * kTile));
-        if (workspace_for(B, Hq, whole) <= kNoAllocScratchBytes) {
-            splits = whole;
-            need = workspace_for(B, Hq, whole);
-        }
-    }
+    // An automatic count is judged by the most splits of two whole tiles per wave, whatever
+    // the format (the array is then used by rule of the sizes alone).  What passes fits: a
+    // format's own count is one, or B H < 256 n at n workgroups per CU, so that it makes
+    // less than 512 n Hq / H records, and n is at most two where Hq / H is eight, four
+    // otherwise: 8192 of the array's 10810.
+    const int whole = std::max(1, std::min(most_splits(B, H, T, kMaxGroupsPerCU), T / (kWaves * 2 * kTile)));
+    const int64_t need = workspace_for(B, Hq, splits > 0 ? resolve_splits(B, H, T, splits, 1, 1) : whole);
     RESKV_REQUIRE(need <= kNoAllocScratchBytes,
                   "reskv_decode_recent_noalloc: these sizes need %lld bytes of split-K scratch; the "
                   "allocation-free entry point holds %lld (use reskv_decode_recent with a workspace)",

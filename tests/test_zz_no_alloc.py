@@ -13,6 +13,7 @@ from oracle import reskv_oracle as o
 from reskv_amd import ResKVKernelConfig, compress
 from reskv_amd import _lib
 from reskv_amd._extension import _rope, cache_descriptors
+from reskv_amd.tensors import CompressedKV
 from tests.gpu_helpers import ATOL, expected_attention, np_, outlier_kv, theta_freq
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +73,24 @@ def test_noalloc_rejects_sizes_beyond_its_scratch(device):
                                            table.data_ptr(), 64, 8, 2, 256, 0, pos, 0.1, 256, None, None, None, 0,
                                            0, None, None)
     assert status != 0 and b"allocation-free" in L.reskv_last_error()
+
+
+@pytest.mark.parametrize("sparsity", [0.5, 0.75])
+@pytest.mark.parametrize("b,h,t", [(169, 2, 400), (350, 2, 200)])
+def test_noalloc_makes_the_splits_of_the_workspace_entry_point_near_its_limit(device, sparsity, b, h, t):
+    """Eight query heads per KV head, so many rows that the largest count of any format would
+    pass the array (three whole shares of T, four rounded up) while the format's own fits."""
+    g = torch.Generator().manual_seed(t)
+    k, v = (torch.randn(b, h, t, 128, generator=g).half().to(device) for _ in range(2))
+    q = torch.randn(b, 8 * h, 1, 128, generator=g).half().to(device)
+    centres = torch.randn(b, h, 8, 128, generator=g).half().to(device)
+    ids = torch.randint(8, (b, h, t), generator=g, dtype=torch.int32).to(device)
+    cache = compress(k, v, ResKVKernelConfig(sparsity=sparsity, num_clusters=8),
+                     clustering=((centres, ids), (centres, ids)))
+    empty = torch.zeros(b, h, 1, 128, dtype=torch.float16, device=device)
+    args = (cache, q, q, empty, empty, theta_freq(), t, 0)
+    ref, got = _call(False, *args), _call(True, *args)
+    assert torch.equal(got, ref)
+    exp = expected_attention(q[:2], CompressedKV(*(x.index_select(torch.arange(2)) for x in (cache.key, cache.value))),
+                             position=t, inv_freq=theta_freq())
+    assert float(np.abs(np_(got[:2]).astype(np.float64) - exp).max()) <= ATOL
