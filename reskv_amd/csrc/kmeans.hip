@@ -102,7 +102,6 @@ struct Problems {
     int32_t* ids[2];       // ids int32 [problems, T]
     uint16_t* out[2];      // final centres fp16 [problems, C, 128]
     int split, vfrom;
-    int vgroup;            // V problems assign by the decode-group rule instead of Lloyd's
 };
 __device__ __forceinline__ int side_of(const Problems& P, long bh) { return bh >= P.split ? 1 : 0; }
 
@@ -264,10 +263,15 @@ __device__ __forceinline__ int sub_of(int j, int e) { return j + (e < 2 ? 4 : 0)
 // increasing order.  A workgroup therefore takes one chunk or a whole part (slots = 4).
 //
 // thi/tlo fp16 [BH, 16 NB, 128] and tnorm fp32 [BH, 16 NB] are the centre
-// tables; psum fp32 [BH, slots, C, 128] and pcnt int [BH, slots, C] (skipped
-// when psum is null).  xnorm (null: formed in place) holds the V tokens' fp16
-// norms [V problems, T]: written when xnorm_new, read otherwise.  LO: some
-// problem has fp32 centres (V problems skip the lo product).
+// tables; psum fp32 [BH, slots, C, 128] and pcnt int [BH, slots, C].  xnorm holds
+// the V tokens' fp16 norms [V problems, T]: written when xnorm_new, read otherwise.
+// LO: some problem has fp32 centres (V problems skip the lo product).
+//
+// SUMS: one Lloyd iteration.  Otherwise the ids alone (decode groups): psum, pcnt
+// and xnorm are null, the V rule is the groups', and a wave takes its sub-tiles in
+// increasing order and ends with the tokens, since a group is a fraction of a chunk
+// (8 problems of 64 tokens, C = 33: K 8.2 -> 7.0 us, V 7.5 -> 6.3; 1024 problems, C = 32:
+// 25.4 -> 23.6 and 26.4 -> 23.1, with one kernel for both purposes before).
 //
 // Bound: reading the rows and the VALU work (argmin, one-hot operands) take about
 // 0.1 ms each per iteration of 256 problems x 8128 tokens and overlap through four
@@ -278,7 +282,7 @@ __device__ __forceinline__ int sub_of(int j, int e) { return j + (e < 2 ? 4 : 0)
 // slower on 512 to 2048 workgroups: 189 against 182 us, 316 against 274.  The kernel
 // before had eight waves reduce 16 KB sums each through LDS for every chunk, wrote
 // a 16 KB partial per 64 KB of tokens, and (C > 32) fitted one workgroup per CU.
-template <int NB, bool LO, int G>
+template <int NB, bool LO, int G, bool SUMS>
 __global__ void __launch_bounds__((Split<NB, G>::threads)) __attribute__((amdgpu_waves_per_eu(4)))
 kmeans_assign_kernel(
     Problems P, const uint16_t* __restrict__ thi, const uint16_t* __restrict__ tlo, const float* __restrict__ tnorm,
@@ -291,7 +295,7 @@ kmeans_assign_kernel(
     constexpr int kSumFloats = CP * kDim;
     constexpr int kSumBytes = G > 1 ? 3 * kSumFloats * 4 : 0;  // r_j handed to group 0 (reuses the rows)
     constexpr int kRowBytes = G * kRows * 2 > kSumBytes ? G * kRows * 2 : kSumBytes;
-    __shared__ __align__(16) uint8_t s_rows[kRowBytes];
+    __shared__ __align__(16) uint8_t s_rows[SUMS ? kRowBytes : 16];
     __shared__ __align__(16) uint4 s_hi[kTab];
     __shared__ __align__(16) uint4 s_lo[LO ? kTab : 1];
     __shared__ __align__(16) uint8_t s_id[G * US * kSub];
@@ -307,8 +311,7 @@ kmeans_assign_kernel(
     const uint16_t* __restrict__ x = P.x[side] + pb * T * kDim;
     int32_t* __restrict__ ids = P.ids[side] + pb * T;
     const bool vrule = bh >= P.vfrom;  // workgroup-uniform
-    const bool vgroup = P.vgroup != 0;
-    float* __restrict__ xn_row = vrule && xnorm != nullptr ? xnorm + (bh - P.vfrom) * T : nullptr;
+    float* __restrict__ xn_row = SUMS && vrule ? xnorm + (bh - P.vfrom) * T : nullptr;
     uint16_t* s_x = reinterpret_cast<uint16_t*>(s_rows) + g * kRows;
     uint8_t* g_id = s_id + g * US * kSub;
 
@@ -332,7 +335,9 @@ kmeans_assign_kernel(
             xr[q] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off + 64 * q, 0, 0));
     };
     // the wave's sub-tile in turn u of a chunk
-    auto sub_in = [&](int u) { return sub_of((u * G + g) * JU + (gw >> 2), gw & 3); };
+    auto sub_in = [&](int u) {
+        return SUMS ? sub_of((u * G + g) * JU + (gw >> 2), gw & 3) : (u * G + g) * US + gw;
+    };
     load_sub(slot, sub_in(0));
 
     // centre operands: lane (col, grp) reads centre nb*16 + col at the same channels,
@@ -368,7 +373,7 @@ kmeans_assign_kernel(
     // ids of the wave's sub-tile at t0 (token rows in xr), staged with its rows
     auto assign_sub = [&](int t0, int k_next, int sub_next) {
         const bool live = t0 + col < T;
-        if (psum != nullptr) {
+        if constexpr (SUMS) {
             // rows past T are zeros, so that they add nothing
             uint4* row = reinterpret_cast<uint4*>(s_x + (gw * kSub + col) * kXPitch + 8 * grp);
 #pragma unroll
@@ -396,11 +401,11 @@ kmeans_assign_kernel(
         }
         float xn = 0.0f;
         if (vrule) {
-            if (xn_row != nullptr && !xnorm_new) {
+            if (SUMS && !xnorm_new) {
                 xn = xn_row[min(t0 + col, T - 1)];
             } else {
                 xn = token_half_norm(xr);
-                if (xn_row != nullptr && grp == 0 && live) xn_row[t0 + col] = xn;
+                if (SUMS && grp == 0 && live) xn_row[t0 + col] = xn;
             }
         }
         load_sub(k_next, sub_next);  // the rows are staged and multiplied: their registers take the next ones
@@ -424,7 +429,7 @@ kmeans_assign_kernel(
             bi += 4 * grp;
             token_argmin(bd, bi);
         } else {
-            if (vgroup) {
+            if constexpr (!SUMS) {
                 // decode groups: fp32(fp16(|x|^2 + |c|^2) - 2 <x, c>), lowest index on
                 // ties, which all centres are for a token whose fp16 norm is infinite
                 float bd = fmaf(-2.0f, acc[0][0], h2f(f2h(xn + cn[0].x)));
@@ -472,8 +477,7 @@ kmeans_assign_kernel(
         }
         // every lane of column col now holds the id of token t0 + col
         if (grp == 0 && live) ids[t0 + col] = bi;
-        if (psum == nullptr) return;
-        if (grp == 0) {
+        if (SUMS && grp == 0) {
             // tokens 4r..4r+3 of all of the unit's sub-tiles are contiguous
             g_id[(col >> 2) * (4 * US) + 4 * gw + (col & 3)] = (uint8_t)(live ? bi & (kMaxClusters - 1) : 0);
             if (live && bi < CP) atomicAdd(&s_cnt[bi], 1);
@@ -517,7 +521,10 @@ kmeans_assign_kernel(
         float4_t tot[MB][NH];
 #pragma unroll
         for (int u = 0; u < W::turns; ++u) {
+            if (!SUMS && k * kChunk + sub_in(u) * kSub >= T) return;  // uniform over the wave; no barrier follows
             assign_sub(k * kChunk + sub_in(u) * kSub, u + 1 < W::turns ? k : k + slots, sub_in((u + 1) % W::turns));
+            // !SUMS, tested at run time in both instances: a chunk's turns in one basic block
+            // are slower (16 problems of 8192, 5 iterations 105 us against 96; 64 with C = 64 350 against 264)
             if (psum == nullptr) continue;
             __syncthreads();  // the unit's rows and ids are staged
 #pragma unroll
@@ -539,7 +546,7 @@ kmeans_assign_kernel(
             __syncthreads();  // the rows are read before the next unit (or the sums) overwrite them
         }
         if constexpr (G == 1) {
-            if (psum != nullptr) {
+            if constexpr (SUMS) {
 #pragma unroll
                 for (int b = 0; b < MB; ++b)
 #pragma unroll
@@ -547,7 +554,7 @@ kmeans_assign_kernel(
             }
         } else {
             // one chunk per workgroup: ((r_0 + r_1) + r_2) + r_3 by group 0
-            if (psum == nullptr) return;
+            if constexpr (!SUMS) return;
             float* sums = reinterpret_cast<float*>(s_rows);  // every group's r_j but group 0's
             auto at = [&](int j, int b, int h, int r) -> float& {
                 return sums[(j - 1) * kSumFloats + (16 * (nb0 + b) + 4 * grp + r) * kDim + d0 + 16 * h + col];
@@ -575,7 +582,7 @@ kmeans_assign_kernel(
             }
         }
     }
-    if (psum == nullptr || g > 0) return;
+    if (!SUMS || g > 0) return;
     float* ps = psum + ((bh * slots) + slot) * (long)C * kDim + d0 + col;
 #pragma unroll
     for (int b = 0; b < MB; ++b)
@@ -705,13 +712,10 @@ struct Tables {
 template <int NB, int G>
 void launch_nb(bool lo, dim3 grid, hipStream_t st, const Problems& P, const Tables& tb, float* psum, int* pcnt,
                float* xnorm, int xnorm_new, int T, int C, int chunks) {
-    const dim3 threads(Split<NB, G>::threads);
-    if (lo)
-        hipLaunchKernelGGL((kmeans_assign_kernel<NB, true, G>), grid, threads, 0, st, P, tb.hi, tb.lo, tb.norm, psum,
-                           pcnt, xnorm, xnorm_new, T, C, chunks);
-    else
-        hipLaunchKernelGGL((kmeans_assign_kernel<NB, false, G>), grid, threads, 0, st, P, tb.hi, tb.lo, tb.norm, psum,
-                           pcnt, xnorm, xnorm_new, T, C, chunks);
+    const auto kernel = psum != nullptr ? (lo ? kmeans_assign_kernel<NB, true, G, true> : kmeans_assign_kernel<NB, false, G, true>)
+                                        : (lo ? kmeans_assign_kernel<NB, true, G, false> : kmeans_assign_kernel<NB, false, G, false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(Split<NB, G>::threads), 0, st, P, tb.hi, tb.lo, tb.norm, psum, pcnt, xnorm,
+                       xnorm_new, T, C, chunks);
 }
 
 int launch_assign(const Problems& P, const Tables& tb, float* psum, int* pcnt, float* xnorm, int xnorm_new, int BH,
@@ -830,7 +834,7 @@ extern "C" int reskv_kmeans_assign(const void* x, const float* centers, int32_t*
     const Layout L = layout(BH, T, C);
     const Tables tb = tables_of(workspace, L);
     const int vfrom = value_mode ? 0 : BH;
-    const Problems P{{(const uint16_t*)x, (const uint16_t*)x}, {ids, ids}, {nullptr, nullptr}, BH, vfrom, 1};
+    const Problems P{{(const uint16_t*)x, (const uint16_t*)x}, {ids, ids}, {nullptr, nullptr}, BH, vfrom};
     hipStream_t st = (hipStream_t)stream;
     if (launch_prep(centers, tb, BH, C, L.Cp, vfrom, st)) return 1;
     return launch_assign(P, tb, nullptr, nullptr, nullptr, 0, BH, T, C, L, st);
@@ -858,7 +862,7 @@ extern "C" int reskv_kmeans(const void* x, const float* centers_init, void* cent
     if (check_pointers(x, workspace)) return 1;
     const uint16_t* xh = (const uint16_t*)x;
     uint16_t* out = (uint16_t*)centers_out;
-    const Problems P{{xh, xh}, {ids, ids}, {out, out}, BH, value_mode ? 0 : BH, 0};
+    const Problems P{{xh, xh}, {ids, ids}, {out, out}, BH, value_mode ? 0 : BH};
     const float* const init[2] = {centers_init, centers_init};
     return run_kmeans(P, init, BH, T, C, iterations, workspace, (hipStream_t)stream);
 }
@@ -876,7 +880,7 @@ extern "C" int reskv_kmeans_kv(const void* k, const void* v, const float* init_k
                   "k-means workspace too small");
     if (check_pointers(k, workspace) || check_pointers(v, workspace)) return 1;
     const Problems P{{(const uint16_t*)k, (const uint16_t*)v}, {ids_k, ids_v}, {(uint16_t*)out_k, (uint16_t*)out_v},
-                     BH, BH, 0};
+                     BH, BH};
     const float* const init[2] = {init_k, init_v};
     return run_kmeans(P, init, 2 * BH, T, C, iterations, workspace, (hipStream_t)stream);
 }
