@@ -48,18 +48,23 @@ def _stream(device):
     return torch._C._cuda_getCurrentRawStream(device.index)
 
 
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_transform_level = torch._C._functorch.maybe_current_level
+_tracing = torch._C._get_tracing_state
+_compiling = torch.compiler.is_compiling
+
+
 def eager():
     """Whether torch runs each operation as it is called, with nothing beside the kernels
     that has to see it: no compilation, tracing, functional transform, forward-mode
     level, and no dispatch or function mode (the default device's concerns new tensors
     only).  A native launch in the place of torch operations on a caller's tensors is one
     that these would miss."""
-    c = torch._C
-    if c._len_torch_function_stack() and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()):
+    if _function_modes() and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()):
         return False
-    return not (c._len_torch_dispatch_stack() or _forward_ad._current_level >= 0
-                or c._functorch.maybe_current_level() is not None or c._get_tracing_state() is not None
-                or torch.compiler.is_compiling())
+    return not (_dispatch_modes() or _forward_ad._current_level >= 0 or _transform_level() is not None
+                or _tracing() is not None or _compiling())
 
 
 def _dev_check(*tensors, contiguous=True):
@@ -604,6 +609,8 @@ def decode_step(query2d, cache, num_q_heads, *, position, start_position, scalin
 
 
 _RING_STRIDES = ctypes.c_int64 * 6
+_Tensor = torch.Tensor
+_increment_version = torch.autograd.graph.increment_version
 
 
 def ring_append(rings, tokens, slot):
@@ -621,32 +628,31 @@ def ring_append(rings, tokens, slot):
     b, h, cap, width = shape
     if width != 128 or not 0 < b * h < 1 << 24 or not 0 <= slot < cap:  # the kernel's own bounds
         return False
-    followed, inference = torch.is_grad_enabled(), torch.is_inference_mode_enabled()
-    pointers, strides, row = [], [], (b, h, 1, 128)
+    row = (b, h, 1, 128)
+    followed, outside = torch.is_grad_enabled(), not torch.is_inference_mode_enabled()
+    strides = []
     for x in tokens:
-        if x.shape != row or x.dtype != dtype or x.get_device() != index or type(x) is not torch.Tensor or x.is_neg():
+        if x.shape != row or x.dtype is not dtype or x.get_device() != index or type(x) is not _Tensor or x.is_neg():
             return False
         sb, sh, _, sd = x.stride()
-        at = x.data_ptr()
-        if sd != 1 or sb % 8 or sh % 8 or at % 16 or (followed and x.requires_grad):
+        if sd != 1 or sb & 7 or sh & 7 or (followed and x.requires_grad):
             return False
         strides += (sb, sh)
-        pointers.append(at)
     for r in rings:  # the kernel indexes all three as dense buffers of one shape
-        at = r.data_ptr()
-        if (r.shape != shape or r.dtype != dtype or r.get_device() != index or type(r) is not torch.Tensor
-                or not r.is_contiguous() or at % 16 or (followed and r.requires_grad)
-                or (r.is_inference() and not inference)):
+        if (r.dtype is not dtype or r.get_device() != index or type(r) is not _Tensor or not r.is_contiguous()
+                or (r is not ring and r.shape != shape) or (outside and r.is_inference())
+                or (followed and r.requires_grad)):
             return False
-        pointers.append(at)
-    k, raw, v, rk, rraw, rv = pointers
     span = b * h * cap * 256
+    (k, raw, v), (rk, rraw, rv) = [x.data_ptr() for x in tokens], [r.data_ptr() for r in rings]
+    if (k | raw | v | rk | rraw | rv) & 15:
+        return False
     for at in (rk, rraw, rv):  # a token that lies in a ring: the copies write one after the other
         if at <= k < at + span or at <= raw < at + span or at <= v < at + span:
             return False
     _lib.check(_lib.lib().reskv_ring_append(k, raw, v, _RING_STRIDES(*strides), rk, rraw, rv, b, h, cap, slot,
                                             _stream(ring.device)), "ring_append")
-    torch.autograd.graph.increment_version(rings)  # as an in-place copy does
+    _increment_version(rings)  # as an in-place copy does
     return True
 
 
