@@ -1,5 +1,6 @@
-// Residual encoders: four lanes per token (eight for 4:16); inputs that are not
-// 16-byte aligned take one wavefront per token, lane L owning channels L and L+64.
+// Residual encoders: four lanes per token (eight for 4:16).  Few rows, rows of a few
+// tokens and inputs that are not 16-byte aligned take one wavefront per token, lane L
+// owning channels L and L+64.
 //
 // Every encoder computes r = f32(x) - f32(c[id]) and ranks channels by the
 // 15-bit magnitude of fp16(r) with ties going to the lower channel index
@@ -779,6 +780,20 @@ bool planes_ok(const EncSides& S, int sides) {
     for (int i = 0; i < sides; ++i) ok = ok && aligned16(S.x[i]) && aligned16(S.cent[i]) && aligned16(S.payload[i]);
     return ok;
 }
+// Whether one wave per token is the faster form of a single-tensor call: its waves do less
+// work one after the other, and four lanes per token leave lanes idle where a (batch,
+// head) row has few tokens.
+//   few: the rows (of 64 tokens) up to which it is, because a wave's latency is all there
+//     is.  2048 rows: INT4 3.8 against 4.4 us, INT2 3.9 / 4.2, structured INT4 3.6 / 3.6, and
+//     at 4096 4.5 / 4.4, 4.5 / 4.2, 4.0 / 3.6; tiles 3.8 / 4.7 and bitmaps 4.1 / 4.7 at
+//     4096 rows, 4.8 / 4.8 and 5.4 / 4.8 at 8192.
+//   most: the tokens of a row from which it is not.  65536 rows of one token: INT4 27
+//     against 85 us, structured INT4 22 / 50, tiles 20 / 108, bitmaps 25 / 98; four lanes
+//     per token take the same for up to 16 tokens, one wave each that many times as long.
+bool one_wave_each(long rows, int T, long few, int most) { return rows <= few || T < most; }
+constexpr long kFewRows16 = 4096, kFewRowsCodes = 2048;
+constexpr int kTokensTiles = 8, kTokensBitmap = 4, kTokensQuant = 4, kTokensSInt4 = 3;
+
 // Calls launch(grid, first (batch, head) row) over all rows: grid y covers at most 65535 of them.
 template <typename Launch>
 int over_rows(int BH, int T, int sides, const char* what, Launch launch) {
@@ -814,7 +829,8 @@ extern "C" int reskv_compress_fp16(const void* keys, const void* centroids, cons
     const EncSides S{{(const uint16_t*)keys, nullptr}, {(const uint16_t*)centroids, nullptr}, {ids, nullptr},
                      {(uint16_t*)payload, nullptr}, {meta, nullptr}, {C, 0}};
     if (tile4_ok(S, 1, nnz)) return launch_tile4(S, 1, B, H, T, struct_index, (hipStream_t)stream);
-    if (planes_ok(S, 1)) return launch_planes<true>(S, 1, B, H, T, nnz, (hipStream_t)stream);
+    if (planes_ok(S, 1) && !one_wave_each(rows, T, kFewRows16, kTokensTiles))
+        return launch_planes<true>(S, 1, B, H, T, nnz, (hipStream_t)stream);
     hipLaunchKernelGGL(encode_qtile_kernel, dim3(grid_for(rows)), dim3(256), 0, (hipStream_t)stream,
                        (const uint16_t*)keys, (const uint16_t*)centroids, ids, (uint16_t*)payload, meta,
                        rows, T, C, nnz, struct_index);
@@ -830,7 +846,8 @@ extern "C" int reskv_compress_bitmap(const void* keys, const void* centroids, co
     const long rows = (long)B * H * T;
     const EncSides S{{(const uint16_t*)keys, nullptr}, {(const uint16_t*)centroids, nullptr}, {ids, nullptr},
                      {(uint16_t*)payload, nullptr}, {meta, nullptr}, {C, 0}};
-    if (planes_ok(S, 1)) return launch_planes<false>(S, 1, B, H, T, nnz, (hipStream_t)stream);
+    if (planes_ok(S, 1) && !one_wave_each(rows, T, kFewRows16, kTokensBitmap))
+        return launch_planes<false>(S, 1, B, H, T, nnz, (hipStream_t)stream);
     hipLaunchKernelGGL(encode_bitmap_kernel, dim3(grid_for(rows)), dim3(256), 0, (hipStream_t)stream,
                        (const uint16_t*)keys, (const uint16_t*)centroids, ids, (uint16_t*)payload, meta,
                        rows, T, C, nnz);
@@ -846,7 +863,8 @@ extern "C" int reskv_compress_quantized(const void* keys, const void* centroids,
     RESKV_REQUIRE(bits == 2 || bits == 4, "quantised encoder requires bits in {2, 4}");
     const long rows = (long)B * H * T;
     // rows read and written with 16-byte (INT2: 8-byte) accesses where they are aligned to them
-    if (aligned16(keys) && aligned16(centroids) && aligned16(qtiles))
+    if (aligned16(keys) && aligned16(centroids) && aligned16(qtiles) &&
+        !one_wave_each(rows, T, kFewRowsCodes, kTokensQuant))
         return over_rows(B * H, T, 1, "encode_quant_kernel", [&](dim3 grid, int bh0) {
             auto kernel = bits == 4 ? encode_quant_kernel<4> : encode_quant_kernel<2>;
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)keys,
@@ -869,7 +887,7 @@ extern "C" int reskv_compress_structured_int4(const void* keys, const void* cent
     if (check_common(keys, centroids, ids, B, H, T, C)) return 1;
     RESKV_REQUIRE(qpacked && qmeta && qscale, "null output pointer");
     const long rows = (long)B * H * T;
-    if (aligned16(keys) && aligned16(centroids))
+    if (aligned16(keys) && aligned16(centroids) && !one_wave_each(rows, T, kFewRowsCodes, kTokensSInt4))
         return over_rows(B * H, T, 1, "encode_sint4_kernel", [&](dim3 grid, int bh0) {
             hipLaunchKernelGGL(encode_sint4_kernel, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)keys,
                                (const uint16_t*)centroids, ids, qpacked, qmeta, (uint16_t*)qscale, T, C, bh0);
@@ -882,7 +900,8 @@ extern "C" int reskv_compress_structured_int4(const void* keys, const void* cent
 
 // A layer's K and V in one launch (grid side dimension); each result equals
 // the single-tensor call's.  Inputs that miss the fast path's alignment run
-// as two single-tensor calls.
+// as two single-tensor calls, and so do many rows of a few tokens (few rows do not:
+// 4096 of them take 4.7 us in one launch of four lanes per token, 6.5 in two).
 extern "C" int reskv_compress_fp16_kv(const void* k, const void* v, const void* k_centroids,
                                       const void* v_centroids, const int32_t* k_ids, const int32_t* v_ids,
                                       void* k_payload, void* v_payload, int32_t* k_meta, int32_t* v_meta, int B,
@@ -890,11 +909,13 @@ extern "C" int reskv_compress_fp16_kv(const void* k, const void* v, const void* 
     if (check_common(k, k_centroids, k_ids, B, H, T, Ck) || check_common(v, v_centroids, v_ids, B, H, T, Cv))
         return 1;
     RESKV_REQUIRE(k_payload && v_payload && k_meta && v_meta, "null output pointer");
+    const long rows = (long)B * H * T;
     const EncSides S{{(const uint16_t*)k, (const uint16_t*)v}, {(const uint16_t*)k_centroids, (const uint16_t*)v_centroids},
                      {k_ids, v_ids}, {(uint16_t*)k_payload, (uint16_t*)v_payload}, {k_meta, v_meta}, {Ck, Cv}};
     if (tile4_ok(S, 2, nnz) && (!struct_index || nnz == 32))
         return launch_tile4(S, 2, B, H, T, struct_index, (hipStream_t)stream);
-    if (planes_ok(S, 2) && !struct_index && nnz > 0 && nnz < kDim && nnz % 8 == 0)
+    if (planes_ok(S, 2) && !struct_index && nnz > 0 && nnz < kDim && nnz % 8 == 0 &&
+        (rows <= kFewRows16 || T >= kTokensTiles))
         return launch_planes<true>(S, 2, B, H, T, nnz, (hipStream_t)stream);
     if (reskv_compress_fp16(k, k_centroids, k_ids, k_payload, k_meta, B, H, T, Ck, nnz, struct_index, stream))
         return 1;
@@ -908,10 +929,12 @@ extern "C" int reskv_compress_bitmap_kv(const void* k, const void* v, const void
     if (check_common(k, k_centroids, k_ids, B, H, T, Ck) || check_common(v, v_centroids, v_ids, B, H, T, Cv))
         return 1;
     RESKV_REQUIRE(k_payload && v_payload && k_meta && v_meta, "null output pointer");
+    const long rows = (long)B * H * T;
     RESKV_REQUIRE(nnz > 0 && nnz <= kDim, "nnz must be in [1, 128]");
     const EncSides S{{(const uint16_t*)k, (const uint16_t*)v}, {(const uint16_t*)k_centroids, (const uint16_t*)v_centroids},
                      {k_ids, v_ids}, {(uint16_t*)k_payload, (uint16_t*)v_payload}, {k_meta, v_meta}, {Ck, Cv}};
-    if (planes_ok(S, 2)) return launch_planes<false>(S, 2, B, H, T, nnz, (hipStream_t)stream);
+    if (planes_ok(S, 2) && (rows <= kFewRows16 || T >= kTokensBitmap))
+        return launch_planes<false>(S, 2, B, H, T, nnz, (hipStream_t)stream);
     if (reskv_compress_bitmap(k, k_centroids, k_ids, k_payload, k_meta, B, H, T, Ck, nnz, stream)) return 1;
     return reskv_compress_bitmap(v, v_centroids, v_ids, v_payload, v_meta, B, H, T, Cv, nnz, stream);
 }
