@@ -16,6 +16,7 @@ that device without synchronising.
 """
 
 import ctypes
+import struct
 import weakref
 from functools import lru_cache
 from types import SimpleNamespace
@@ -42,6 +43,9 @@ def _require(cond, msg):
 
 def _ptr(t):
     return None if t is None or t.numel() == 0 else t.data_ptr()
+
+
+_Tensor = torch.Tensor
 
 
 def _stream(device):
@@ -580,7 +584,8 @@ def decode_step(query2d, cache, num_q_heads, *, position, start_position, scalin
     dev = query2d.device
     index = query2d.get_device()
     for x in cache.key._native + cache.value._native:
-        _require(x is None or x.get_device() == index, "all tensors must be on the same GPU")
+        if x is not None and x.get_device() != index:
+            raise RuntimeError("all tensors must be on the same GPU")
     _require(query2d.is_cuda, "all tensors must be on the same GPU")
     if recent is not None:
         _dev_check(query2d, *recent)
@@ -593,7 +598,8 @@ def decode_step(query2d, cache, num_q_heads, *, position, start_position, scalin
     nh, t, splits = int(num_q_heads), cache.seq_len, int(splits)
     freq, table = _rope(inv_freq, rope_theta, dev, int(start_position) + t)
     L = _lib.lib()
-    out = _empty((b * nh, 128), torch.float16, dev)  # plain, also for a subclass's query
+    # plain, also for a subclass's query
+    out = torch.empty_like(query2d) if type(query2d) is _Tensor else _empty((b * nh, 128), torch.float16, dev)
     ws = _workspace(L.reskv_decode_workspace_bytes(b, nh, kh, t, splits), dev)
     common = (query2d.data_ptr(), _descriptor(cache.key), _descriptor(cache.value), freq.data_ptr(),
               table.data_ptr(), b, nh, kh, t, int(start_position), int(position), float(scaling), splits)
@@ -608,8 +614,7 @@ def decode_step(query2d, cache, num_q_heads, *, position, start_position, scalin
     return out
 
 
-_RING_STRIDES = ctypes.c_int64 * 6
-_Tensor = torch.Tensor
+_RING_STRIDES = struct.Struct("6q").pack
 _increment_version = torch.autograd.graph.increment_version
 
 
@@ -651,7 +656,7 @@ def ring_append(rings, tokens, slot):
         if at <= k < at + span or at <= raw < at + span or at <= v < at + span:
             return False
     _lib.check(_lib.lib().reskv_ring_append(k, raw, v, _RING_STRIDES(*strides), rk, rraw, rv, b, h, cap, slot,
-                                            _stream(ring.device)), "ring_append")
+                                            torch._C._cuda_getCurrentRawStream(index)), "ring_append")
     _increment_version(rings)  # as an in-place copy does
     return True
 

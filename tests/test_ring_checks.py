@@ -27,7 +27,7 @@ def append(monkeypatch):
 
     monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
     monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: -1, raising=False)
-    monkeypatch.setattr(_extension, "_stream", lambda d: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda d: 0, raising=False)
     monkeypatch.setattr(_extension._lib, "lib", lambda: Library())
 
     def call(rings, tokens, slot=0):
