@@ -480,8 +480,9 @@ __device__ __forceinline__ void residual_f(const StageView<F>& S, const Prefetch
 // biased to unsigned fields by flipping their sign bits (u = code + 2^(bits-1)).
 // Two instructions a pair and two a word; pairs of neighbours, byte permutes under a
 // 0x64 high byte, a mask and a packed FMA, took three a pair and one a word.  29 of 330
-// VALU instructions a tile; B = 8, T = 16384, INT4: 65.3 -> 64.7 us (the VALU is busy
-// 69% of the time, the LDS 53%, the matrix cores 17%).
+// VALU instructions a tile; B = 8, T = 16384, INT4: 65.3 -> 64.7 us (of the cycles
+// counted, the VALU is busy in 69%, matrix-core issue included, the LDS in 53%, 46% of
+// that bank conflicts, and the matrix cores in 17%).
 template <int F>
 __device__ __forceinline__ void code_halves(const StageView<F>& S, const Prefetch<F>& R, int t, int g, uint32_t* h) {
     uint32_t lw[4];

@@ -396,7 +396,7 @@ __device__ __forceinline__ uint32_t select_tiles(const uint32_t* pl, int per_til
 // 8 heads x 8192 tokens, K and V in one launch: 50% bitmap 18.7 -> 15.6 us, 75%
 // 17.9 -> 13.9 us (byte planes before), 50% tiles 41.2 -> 16.2 us (one wave per
 // token before).  64 heads x 16384 tokens: 231 -> 193, 210 -> 169 and 503 ->
-// 208 us, i.e. 4.4, 4.4 and 4.1 TB/s (a large copy reaches 4.9).
+// 208 us, i.e. 4.4, 4.2 and 4.1 TB/s (a large copy reaches 4.9).
 template <bool TILE, int NNZ>
 __global__ void __launch_bounds__(256) encode_planes_kernel(EncSides S, int T, int nnz_arg, int bh0) {
     __shared__ __align__(16) uint16_t s_rows[kWavesPerBlock][kRowHalves + kWave];
@@ -598,7 +598,7 @@ __global__ void __launch_bounds__(256) encode_quant_kernel(const uint16_t* __res
 // Structured INT4 (compression.cu:153-239): 1 of every 4 channels, four lanes
 // per token as above (lane q: subgroups 8 q .. 8 q + 7, i.e. payload word q and
 // half a metadata word), so every load and store is a contiguous run.  K and V
-// of 64 heads x 16384 tokens: 541 -> 128 us, 4.8 TB/s, the rate of a large copy.
+// of 64 heads x 16384 tokens: 541 -> 128 us, 4.7 TB/s (a large copy reaches 4.9).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) encode_sint4_kernel(const uint16_t* __restrict__ keys,
                                                            const uint16_t* __restrict__ cent,

@@ -34,8 +34,9 @@
 // and tokens are exact in fp16 and the products accumulate in fp32, in an order
 // that does not depend on the launch; counts are integer LDS adds.  Sums, counts
 // and centres are deterministic, and equal for paired and separate runs.
-// Update (kmeans_update_kernel): one workgroup per (cluster, problem) adds the
-// partials in a fixed order, writes the new centre and its tables.
+// Update (kmeans_update_kernel): a workgroup adds the partials of four clusters of a
+// problem, or of one where there are more than four partials, in a fixed order, and
+// writes the new centres and their tables.
 #include "common.h"
 #include "../../include/reskv_hip.h"
 using namespace reskv;

@@ -49,8 +49,9 @@ struct AttnArgs {
 // Bound: matrix cores and LDS together.  A wave issues 32 products of 32 cycles per
 // tile and reads 32 KB of LDS, and four waves of a CU's two workgroups share 128
 // bytes a cycle of it, so both take about 1024 cycles; the softmax of the other
-// workgroup runs beside them.  32 / 8 heads, one prompt: 1024 tokens 32 us, 4096
-// 205 us (672 TFLOP/s over the causal half), 8192 622 us (884 TFLOP/s); in torch (two
+// workgroup runs beside them.  32 / 8 heads, one prompt, back to back: 1024 tokens 31 us,
+// 4096 179 us (768 TFLOP/s over the causal half), 8192 632 us (869 TFLOP/s), and 230 us at
+// 4096 within a prompt pass, after the projections; in torch (two
 // matrix products with fp32 scores, mask and softmax passes between them) a prompt of
 // 4096 took about 4 ms.
 template <int HPW>
