@@ -297,7 +297,7 @@ class RandomLlama:
         b, t = ids.shape
         cos, sin = self.rope_tables(t)
         x = self.embed[ids]  # [B, T, hidden]
-        fused = self._fused(t)
+        fused = b > 0 and self._fused(t)
         rep = s.heads // s.kv_heads
         causal = None if fused else torch.ones(q_rows, t, dtype=torch.bool, device=self.device)
         for li, p in enumerate(self.layers):

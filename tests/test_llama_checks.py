@@ -122,3 +122,13 @@ def test_norm_gains_that_the_kernel_refuses_take_the_torch_formulas(name, gains)
     assert model._fused(64)
     model.layers[1][name] = gains
     assert not model._fused(64)
+
+
+def test_an_empty_batch_of_prompts_takes_the_torch_formulas(monkeypatch):
+    shape = LlamaShape(layers=1, hidden=256, heads=2, kv_heads=1, ffn=64, vocab=50)
+    model = RandomLlama(shape, "cpu")
+    ids = torch.zeros(0, 5, dtype=torch.int64)
+    want = model.prefill(ids, lambda *a: None, logits=True)
+    assert want.shape == (0, 50)
+    monkeypatch.setattr(RandomLlama, "_fused", lambda self, t: True)
+    assert model.prefill(ids, lambda *a: None, logits=True).shape == (0, 50)
