@@ -293,8 +293,8 @@ kmeans_assign_kernel(
     constexpr int CP = NB * 16, MB = W::MB, NH = W::NH, JU = W::JU, US = W::US;
     constexpr int kTab = CP * kDim / 8;                 // 16-byte slots of a centre table
     constexpr int kRows = US * kSub * kXPitch;          // halves of a group's staged rows
-    constexpr int kSumFloats = CP * kDim;
-    constexpr int kSumBytes = G > 1 ? 3 * kSumFloats * 4 : 0;  // r_j handed to group 0 (reuses the rows)
+    constexpr int kSumPitch = kDim + 4;  // floats: the four rows that a wave writes at once on different banks
+    constexpr int kSumBytes = G > 1 ? 4 * CP * kSumPitch * 4 : 0;  // the groups' r_j (reuse the rows)
     constexpr int kRowBytes = G * kRows * 2 > kSumBytes ? G * kRows * 2 : kSumBytes;
     __shared__ __align__(16) uint8_t s_rows[SUMS ? kRowBytes : 16];
     __shared__ __align__(16) uint4 s_hi[kTab];
@@ -554,36 +554,32 @@ kmeans_assign_kernel(
                     for (int h = 0; h < NH; ++h) part[b][h] += tot[b][h];
             }
         } else {
-            // one chunk per workgroup: ((r_0 + r_1) + r_2) + r_3 by group 0
+            // one chunk per workgroup: ((r_0 + r_1) + r_2) + r_3, by all threads from LDS
             if constexpr (!SUMS) return;
-            float* sums = reinterpret_cast<float*>(s_rows);  // every group's r_j but group 0's
-            auto at = [&](int j, int b, int h, int r) -> float& {
-                return sums[(j - 1) * kSumFloats + (16 * (nb0 + b) + 4 * grp + r) * kDim + d0 + 16 * h + col];
-            };
-            if (g > 0) {
+            float* sums = reinterpret_cast<float*>(s_rows);
 #pragma unroll
-                for (int b = 0; b < MB; ++b)
+            for (int b = 0; b < MB; ++b)
 #pragma unroll
-                    for (int h = 0; h < NH; ++h)
+                for (int h = 0; h < NH; ++h)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) at(g, b, h, r) = tot[b][h][r];
-            }
+                    for (int r = 0; r < 4; ++r)
+                        sums[(g * CP + 16 * (nb0 + b) + 4 * grp + r) * kSumPitch + d0 + 16 * h + col] = tot[b][h][r];
             __syncthreads();
-            if (g == 0) {
+            float4* ps = reinterpret_cast<float4*>(psum + ((bh * slots) + slot) * (long)C * kDim);
+            for (int i = tid; i < C * (kDim / 4); i += W::threads) {
+                const float* src = sums + (i >> 5) * kSumPitch + 4 * (i & 31);
+                float4 v[4];
 #pragma unroll
-                for (int b = 0; b < MB; ++b)
-#pragma unroll
-                    for (int h = 0; h < NH; ++h) {
-#pragma unroll
-                        for (int j = 1; j < 4; ++j)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) tot[b][h][r] += at(j, b, h, r);
-                        part[b][h] += tot[b][h];
-                    }
+                for (int j = 0; j < 4; ++j) v[j] = *reinterpret_cast<const float4*>(src + j * CP * kSumPitch);
+                // from zero as the parts are, so that a sum of negative zero has their sign
+                auto add = [](float a, float b, float c, float d) { return 0.5f * (0.0f + (((a + b) + c) + d)); };
+                ps[i] = make_float4(add(v[0].x, v[1].x, v[2].x, v[3].x), add(v[0].y, v[1].y, v[2].y, v[3].y),
+                                    add(v[0].z, v[1].z, v[2].z, v[3].z), add(v[0].w, v[1].w, v[2].w, v[3].w));
             }
+            for (int i = tid; i < C; i += W::threads) pcnt[(bh * slots + slot) * C + i] = s_cnt[i];
         }
     }
-    if (!SUMS || g > 0) return;
+    if (!SUMS || G > 1) return;
     float* ps = psum + ((bh * slots) + slot) * (long)C * kDim + d0 + col;
 #pragma unroll
     for (int b = 0; b < MB; ++b)
@@ -725,7 +721,8 @@ int launch_assign(const Problems& P, const Tables& tb, float* psum, int* pcnt, f
     const bool lo = P.vfrom > 0;
     // a chunk's sub-tiles over 16 waves instead of four turns of four while the
     // grid leaves CUs idle (C = 32, 10 iterations: 64 workgroups 117 against 131 us,
-    // 256 134 against 149, 384 192 against 165)
+    // 256 134 against 149, 384 192 against 165; with the groups' sums added by all threads
+    // since, the first figures are 6 us less)
     const bool wide = L.slots == L.chunks && (int64_t)L.chunks * BH <= kCUs;
     switch (L.Cp / 16) {
     case 1:
