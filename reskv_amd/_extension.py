@@ -465,12 +465,13 @@ def _described(t):
     """What a CompressedTensor's native views are to the library, without their
     addresses: (format, bits, centroids, width, token row stride, centroid row
     stride, has metadata, has scale).  It follows from the views, which are made and
-    checked with the tensor, and from the plan, and is worked out again when either
-    has been replaced."""
+    checked with the tensor, and from the plan, and is worked out again, and the views'
+    devices compared, when either has been replaced."""
     known = t.__dict__.get("_layout")
     if known is not None and known[0] is t._native and known[1] is t.plan:
         return known[2]
     c, i, p, m, sc = t._native
+    _require(all(x is None or x.device == p.device for x in t._native), "all tensors must be on the same GPU")
     plan = t.plan
     if plan.bits == 16 and plan.layout == "unstructured":
         fmt, bits, sc = _lib.FMT_BITMAP, 16, None
@@ -583,10 +584,8 @@ def decode_step(query2d, cache, num_q_heads, *, position, start_position, scalin
     """
     dev = query2d.device
     index = query2d.get_device()
-    for x in cache.key._native + cache.value._native:
-        if x is not None and x.get_device() != index:
-            raise RuntimeError("all tensors must be on the same GPU")
-    _require(query2d.is_cuda, "all tensors must be on the same GPU")
+    _require(query2d.is_cuda and cache.key._native[2].get_device() == index
+             and cache.value._native[2].get_device() == index, "all tensors must be on the same GPU")
     if recent is not None:
         _dev_check(query2d, *recent)
     if torch._C._cuda_getDevice() != index:
@@ -601,6 +600,7 @@ def decode_step(query2d, cache, num_q_heads, *, position, start_position, scalin
     # plain, also for a subclass's query
     out = torch.empty_like(query2d) if type(query2d) is _Tensor else _empty((b * nh, 128), torch.float16, dev)
     ws = _workspace(L.reskv_decode_workspace_bytes(b, nh, kh, t, splits), dev)
+    # (a tensor's views share a device: _described)
     common = (query2d.data_ptr(), _descriptor(cache.key), _descriptor(cache.value), freq.data_ptr(),
               table.data_ptr(), b, nh, kh, t, int(start_position), int(position), float(scaling), splits)
     if recent is None:
