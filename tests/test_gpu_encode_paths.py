@@ -1,7 +1,9 @@
 """The encoders that work on bit planes (four lanes per token) against the
 one-wave-per-token kernels that inputs off the 16-byte alignment still take:
 the same bytes for every format, also for residuals that are not finite, for
-subnormal and overflowing scales, and for quotients on rounding boundaries."""
+subnormal and overflowing scales, and for quotients on rounding boundaries.
+At these row counts an aligned call takes the one-wave kernels too; the same inputs
+at the counts that take the bit planes are in test_gpu_encode_rows.py."""
 
 import pytest
 import torch
