@@ -627,7 +627,9 @@ def ring_append(rings, tokens, slot):
     something has to see."""
     ring = rings[0]
     index = ring.get_device()
-    if not ring.is_cuda or ring.element_size() != 2 or torch._C._cuda_getDevice() != index or not eager():
+    # (the device query last: a host that follows fake tensors may have no GPU)
+    if (not ring.is_cuda or ring.element_size() != 2 or not eager() or type(ring) is not _Tensor
+            or torch._C._cuda_getDevice() != index):
         return False
     shape, dtype = ring.shape, ring.dtype
     b, h, cap, width = shape

@@ -139,3 +139,16 @@ def test_reorder_and_crop(monkeypatch):
     with pytest.raises(NotImplementedError):
         c.crop(3)
     assert c.get_seq_length() == 40 and len(c) == 2
+
+
+def test_fake_tensors_pass_through_a_layer_without_a_gpu():
+    """Shapes are worked out for GPU tensors on a host that has none (no native call, no device query)."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    with FakeTensorMode():
+        layer = ResKVLayerCache(ResKVKernelConfig(sparsity=0.75))
+        prompt = torch.zeros(2, 2, 5, 128, dtype=torch.float16, device="cuda")
+        layer.update(prompt, prompt, {"raw_keys": prompt})
+        token = prompt[:, :, :1]
+        keys, values = layer.update(token, token, {"raw_keys": token})
+        assert keys.shape == values.shape == (2, 2, 6, 128) and keys.is_cuda
