@@ -56,7 +56,6 @@ _dispatch_modes = torch._C._len_torch_dispatch_stack
 _function_modes = torch._C._len_torch_function_stack
 _transform_level = torch._C._functorch.maybe_current_level
 _tracing = torch._C._get_tracing_state
-_compiling = torch.compiler.is_compiling
 
 
 def eager():
@@ -65,10 +64,12 @@ def eager():
     level, and no dispatch or function mode (the default device's concerns new tensors
     only).  A native launch in the place of torch operations on a caller's tensors is one
     that these would miss."""
+    if torch.compiler.is_compiling():  # first: a compiler follows no further
+        return False
     if _function_modes() and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()):
         return False
     return not (_dispatch_modes() or _forward_ad._current_level >= 0 or _transform_level() is not None
-                or _tracing() is not None or _compiling())
+                or _tracing() is not None)
 
 
 def _dev_check(*tensors, contiguous=True):
@@ -626,10 +627,10 @@ def ring_append(rings, tokens, slot):
     inference tensors outside inference mode (which the copies refuse), or a call that
     something has to see."""
     ring = rings[0]
+    if not ring.is_cuda or ring.element_size() != 2 or not eager() or type(ring) is not _Tensor:
+        return False
     index = ring.get_device()
-    # (the device query last: a host that follows fake tensors may have no GPU)
-    if (not ring.is_cuda or ring.element_size() != 2 or not eager() or type(ring) is not _Tensor
-            or torch._C._cuda_getDevice() != index):
+    if torch._C._cuda_getDevice() != index:  # (last: a host that follows fake tensors may have no GPU)
         return False
     shape, dtype = ring.shape, ring.dtype
     b, h, cap, width = shape

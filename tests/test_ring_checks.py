@@ -156,3 +156,12 @@ def test_tokens_that_lie_in_a_ring_are_left_to_torch(append):
     rings, tokens = _rings(), _tokens()
     tokens[1] = rings[0][:, :, 3:4]
     assert not append(rings, tokens, 3)
+
+
+def test_a_compiled_call_takes_the_other_path_in_one_graph():
+    """torch.compile follows the question itself without a graph break."""
+    def which(x):
+        return x + (1.0 if _extension.eager() else 2.0)
+
+    assert torch.compile(which, backend="eager", fullgraph=True)(torch.zeros(2)).tolist() == [2.0, 2.0]
+    assert which(torch.zeros(2)).tolist() == [1.0, 1.0]
