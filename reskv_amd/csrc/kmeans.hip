@@ -433,13 +433,13 @@ kmeans_assign_kernel(
             if constexpr (!SUMS) {
                 // decode groups: fp32(fp16(|x|^2 + |c|^2) - 2 <x, c>), lowest index on
                 // ties, which all centres are for a token whose fp16 norm is infinite
-                float bd = fmaf(-2.0f, acc[0][0], h2f(f2h(xn + cn[0].x)));
-                bi = 0;
+                constexpr int kNone = 1 << 20;
+                float bd = INFINITY;
+                bi = kNone;
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        if (nb == 0 && r == 0) continue;
                         const float e = h2f(f2h(xn + cnorm(cn[nb], r)));
                         const float d = fmaf(-2.0f, acc[nb][r], e);
                         const bool take = d < bd;
@@ -448,6 +448,7 @@ kmeans_assign_kernel(
                     }
                 bi += 4 * grp;
                 token_argmin(bd, bi);
+                bi = bi >= kNone ? 0 : bi;
             } else {
                 // Lloyd: fp16 cdist.  The winner is the lowest index whose fp16
                 // root equals the smallest one: with dmin the smallest fp16

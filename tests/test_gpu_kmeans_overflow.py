@@ -58,3 +58,25 @@ def test_appended_groups_are_decoded_with_the_centroid_that_they_were_encoded_wi
         err = np.abs(whole - np_(x).astype(np.float64))[kept]
         # one rounding of the residual to fp16: half a unit in the last place of at most 512
         assert kept.mean() > 0.45 and err.max() <= 0.25
+
+
+@pytest.mark.parametrize("count", [16, 33])
+def test_centres_without_a_distance_are_passed_over(device, count):
+    """A NaN centre is nobody's nearest one, wherever it stands in a lane's scan; a token
+    without any finite distance takes the lowest index."""
+    g = seeded(count)
+    x = torch.randn(2, 70, 128, generator=g).half()
+    centres = torch.randn(2, count, 128, generator=g).half()
+    nan = [0, 4, 5, 15, count - 1]
+    clean = np_(centres).copy()
+    centres[:, nan, 3] = float("nan")
+    x[:, 9] = float("nan")
+    ids = np_(kmeans_assign(x.to(device), centres.float().to(device), value=True))
+    d = o.incremental_value_distances(np_(x), clean)
+    d[:, :, nan] = np.inf
+    finite = np.isfinite(d).any(-1) & ~np.isnan(d).any(-1)
+    assert not finite[:, 9].any() and finite.sum() == 2 * 69
+    assert (ids[:, 9] == 0).all() and not np.isin(ids[finite], nan).any()
+    got = np.take_along_axis(d, ids[..., None].astype(np.int64), -1)[..., 0][finite]
+    # an fp16 norm that rounds the other way moves a distance by two fp16 steps of at most 512
+    assert (got - d.min(-1)[finite] <= 4 * 0.25).all()
